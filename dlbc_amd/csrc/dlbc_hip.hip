@@ -125,12 +125,12 @@ void apply_block_order(dlbc_gpu_ctx *c, int chunk) {
 // ---- population loaders -----------------------------------------------------
 // A loader returns population i of component f at site s in FP64: the stored
 // value (FP64 storage) or w_i rho0_f + the stored deviation (shifted storage).
+template <int Q>
 struct LoadF64 {
   const double *A;
   int64_t sp;
-  int q;
   __device__ double operator()(int f, int i, int s) const {
-    return A[(int64_t)(f * q + i) * sp + s];
+    return A[pop_elem_f64<Q>(f, i, s, sp)];
   }
 };
 template <class St>
@@ -589,11 +589,13 @@ struct AdvectOnly {
 template <class Fn>
 int with_loader(dlbc_gpu_ctx *c, Fn fn) {
   if (c->storage == DLBC_STORAGE_F64) {
-    const LoadF64 ld{static_cast<const double *>(c->popA), c->geo.sp, c->q};
-    if (c->d == 3) return fn(D3Q19{}, ld);
-    if (c->d == 2) return fn(D2Q9{}, ld);
-    if (c->q == 5) return fn(D1Q5{}, ld);
-    return fn(D1Q3{}, ld);
+    auto go = [&](auto lat) {
+      return fn(lat, LoadF64<decltype(lat)::q>{static_cast<const double *>(c->popA), c->geo.sp});
+    };
+    if (c->d == 3) return go(D3Q19{});
+    if (c->d == 2) return go(D2Q9{});
+    if (c->q == 5) return go(D1Q5{});
+    return go(D1Q3{});
   }
   if (c->storage == DLBC_STORAGE_F32_SHIFT) {
     const LoadShift<float> ld{static_cast<const float *>(c->popA), c->geo.sp,
@@ -1831,7 +1833,7 @@ int batch_prepare(dlbc_batch *b) {
 // offsets (the OFF32 variants).
 bool batch_off32(const dlbc_batch *b) {
   for (auto *c : b->ctx)
-    if (!split_off32(c->geo)) return false;
+    if (!shift_off32(c->geo, c->elem)) return false;
   return true;
 }
 

@@ -117,7 +117,7 @@ __device__ __forceinline__ void batch_tile(const BatchItem &item, ConstLattice &
     const int ring = FULL ? Sh::ring : 2 * (vz + 2) + 2 * vy;
     const int ring_items = ring * 2 * Q;
     const int y = y0 + ly, z = z0 + lz;
-    // component f's populations: elements shift_elem(f, i, s) = 2 (i sp + s) + f
+    // component f's populations: elements shift_elem(f, i, s)
     const Store *__restrict__ Af = A + f;
     Store *__restrict__ Wf = W + f;
     const float rho0 = pl.rho0;
@@ -142,7 +142,7 @@ __device__ __forceinline__ void batch_tile(const BatchItem &item, ConstLattice &
         const bool bb = (sw >> L::bounce[i]) & 1u;
         const int comp = bb ? L::bounce[i] : i;
         const int src = bb ? self : gsite(sx, sy, sz);
-        n[i] = to_f(Af[2 * ((int64_t)comp * sp + src)]);
+        n[i] = to_f(Af[2 * (64 * comp + tile_elem<19>(src))]);
       }
     };
     auto drho = [](const float *n) { return shifted_drho(n); };
@@ -249,7 +249,7 @@ __device__ __forceinline__ void batch_tile(const BatchItem &item, ConstLattice &
                                      wrapf(z + L::c[i][2], nz));
                 return B.P[f * sp + (b ? nb : s)];  // the density at solid sites
               },
-              [&](int i, float v) { store_nt<Store>(&Wf[2 * ((int64_t)i * sp + s)], v); });
+              [&](int i, float v) { store_nt<Store>(&Wf[2 * (64 * i + tile_elem<19>(s))], v); });
         }
       }
 #pragma unroll

@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(64 * TY)
       const bool bb = SOLID && ((sw >> L::bounce[i]) & 1u);
       const int comp = bb ? L::bounce[i] : i;
       const int src = bb ? self : gsite(sx, sy, sz);
-      n[i] = Af[(int64_t)comp * sp + src];
+      n[i] = Af[64 * comp + tile_elem<Q>(src)];
     }
   };
   // Stage the streamed populations of the ring sites of plane x.
@@ -186,7 +186,7 @@ __global__ void __launch_bounds__(64 * TY)
         const bool bb = (rw >> bi) & 1u;
         const int comp = bb ? bi : i;
         const int src = bb ? self : gsite(wrapf(x - cx, nx), wrapf(yy - cy, ny), wrapf(zz - cz, nz));
-        v = A[(int64_t)(fr * Q + comp) * sp + src];
+        v = A[pop_elem_f64<Q>(fr, comp, src, sp)];
       }
       stg[w] = v;
     }
@@ -284,7 +284,7 @@ __global__ void __launch_bounds__(64 * TY)
                              [&](int i, double v) {
                                // streaming store: the new populations are not read again
                                // in this step, so they bypass the caches
-                               __builtin_nontemporal_store(v, &Bf[(int64_t)i * sp + s]);
+                               __builtin_nontemporal_store(v, &Bf[64 * i + tile_elem<Q>(s)]);
                              });
       }
     }

@@ -30,13 +30,13 @@ __device__ inline St to_storage(double v, int i, double rho0) {
   }
 }
 
-// Element of population i of component f at site s: FP64 storage is
-// [C][q][sp]; shifted storage keeps the two components side by side
+// Element of population i of component f at site s: FP64 storage keeps a
+// component's tiles in turn; shifted storage keeps the two components side by side
 // (shift_elem).
 template <class St>
 __device__ inline int64_t pop_elem(int f, int i, int s, int q, int64_t sp) {
   if constexpr (std::is_same<St, double>::value)
-    return (int64_t)(f * q + i) * sp + s;
+    return f * (q * sp) + (int64_t)(s >> 6) * (64 * q) + 64 * i + (s & 63);
   else
     return shift_elem(f, i, s, sp);
 }

@@ -67,36 +67,37 @@ __device__ inline T *lane_elem(T *base, int64_t k) {
   }
 }
 
+// Site row + z of a row that starts at site `row` (wave-uniform): the scalar base
+// of the row's first tile plus the lane's place from there (fo: the component's
+// first element).
+template <bool OFF32, class T>
+__device__ inline T *row_elem(T *base, int row, int64_t fo, int z) {
+  return lane_elem<OFF32>(base + tile_elem<19>(row & ~63), fo + tile_elem<19>((row & 63) + z));
+}
+
 // The 19 streamed populations of component f at site (x, y, z) -- row bases
 // rb[dx+1][dy+1] = site index of (x+dx, y+dy, 0), wrapped; z offsets zm/zp of
 // this lane -- with bounce-back by the solid word sw (advection.d:61-89).
 // Every address is a wave-uniform base (population and row) plus a 32-bit
-// lane offset (component f's arrays start at f 19 sp, then the z position);
-// without solids the lane offsets are the same three values for every
-// population, so the compiler keeps three registers, not 19 addresses.
+// lane offset (component f's arrays start at f 19 sp, then the z position).
 template <bool SOLID, bool OFF32>
 __device__ inline void march_pull(const double *__restrict__ A, const Geo &g, int f,
                                   const int (&rb)[3][3], int z, int zm, int zp, uint32_t sw,
                                   double *n) {
   using L = D3Q19;
-  const uint32_t fo = (uint32_t)f * 19u * (uint32_t)g.sp;
-  const uint32_t lz[3] = {fo + (uint32_t)zp, fo + (uint32_t)z, fo + (uint32_t)zm};
+  const int64_t fo = (int64_t)f * 19 * g.sp;
+  const int lz[3] = {zp, z, zm};
 #pragma unroll
   for (int i = 0; i < L::q; ++i) {
     const int cz = L::c[i][2];
     const int rs = rb[1 - L::c[i][0]][1 - L::c[i][1]];
     if (SOLID) {
-      // a base below both candidate elements: population min(i, bounce(i))
-      // of row min(rs, own row); the lane picks its offset from it
-      const int b = L::bounce[i], mc = i < b ? i : b;
-      const int r0 = rb[1][1];
-      const int mr = rs < r0 ? rs : r0;
-      const double *base = A + (int64_t)mc * g.sp + mr;
-      const uint32_t on = (uint32_t)((i - mc) * g.sp + (rs - mr)) + lz[cz + 1];
-      const uint32_t ob = (uint32_t)((b - mc) * g.sp + (r0 - mr)) + lz[1];
-      n[i] = *lane_elem<OFF32>(base, ((sw >> b) & 1u) ? ob : on);
+      const int b = L::bounce[i];
+      const double *on = row_elem<OFF32>(A + 64 * i, rs, fo, lz[cz + 1]);
+      const double *ob = row_elem<OFF32>(A + 64 * b, rb[1][1], fo, lz[1]);
+      n[i] = *(((sw >> b) & 1u) ? ob : on);
     } else {
-      n[i] = *lane_elem<OFF32>(A + (int64_t)i * g.sp + rs, lz[cz + 1]);
+      n[i] = *row_elem<OFF32>(A + 64 * i, rs, fo, lz[cz + 1]);
     }
   }
 }
@@ -166,12 +167,9 @@ __device__ inline void march_collide(double (*ring)[RY][2][NZ + 2], int sl, int 
   if (p.eq_form == kBDist2)
     weighted_velocity<L, 2>([&](int ff, int d) { return ff == f ? mom[d] : mom_p[d]; }, total, p,
                             wv);
-  // element f 19 sp + i sp + s of B: the scalar base of population i in this
-  // row plus the lane offset f 19 sp + z
-  const uint32_t lo = (uint32_t)f * 19u * (uint32_t)g.sp + (uint32_t)z;
-  double *__restrict__ Brow = B + rb[1][1];
+  const int64_t fo = (int64_t)f * 19 * g.sp;
   collide_d3q19_streamed(f, nc, rho, total, F, wv, p, [&](int i, double v) {
-    __builtin_nontemporal_store(v, lane_elem<OFF32>(Brow + (int64_t)i * g.sp, lo));
+    __builtin_nontemporal_store(v, row_elem<OFF32>(B + 64 * i, rb[1][1], fo, z));
   });
 }
 
@@ -344,10 +342,8 @@ inline void launch_march_nw(const double *A, double *B, const uint32_t *nbw, con
 #undef DLBC_MARCH_LAUNCH
 }
 
-// Lane offsets of the march kernel, in elements: below 27 sp in the pulls
-// with bounce-back (up to 7 sp between a population and its bounce partner,
-// one row span, the component's 19 sp), below 20 sp elsewhere.  OFF32 when
-// 28 sp fits 2^29 (byte offsets below 2^32).
+// Lane offsets of the march kernel, in elements: the component's 19 sp and a
+// row.  OFF32 when 28 sp fits 2^29 (byte offsets below 2^32).
 inline bool march_off32(const Geo &g) { return 28 * g.sp < ((int64_t)1 << 29); }
 
 // Whether the march schedule serves a lattice with `ty` z-rows per workgroup

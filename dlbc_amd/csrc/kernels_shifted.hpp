@@ -80,10 +80,11 @@ __device__ inline void store_nt<__half>(__half *p, float v) {
 }
 
 // Layout of a shifted-storage buffer: the two components of a population sit
-// side by side, element (f, i, s) at 2 (i sp + s) + f, so one 8-byte (FP32)
-// or 4-byte (FP16) access moves both components of a site.
+// side by side, element (f, i, s) at 2 ((s / 64 * 19 + i) 64 + s % 64) + f (the
+// tiles of kernels_twopass.hpp), so one 8-byte (FP32) or 4-byte (FP16) access
+// moves both components of a site.
 __host__ __device__ inline int64_t shift_elem(int f, int i, int64_t s, int64_t sp) {
-  return 2 * ((int64_t)i * sp + s) + f;
+  return 2 * (64 * (int64_t)i + tile_elem<19>(s)) + f;
 }
 
 // Both components at p (an even element) as FP32.

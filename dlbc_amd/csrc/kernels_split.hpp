@@ -96,8 +96,8 @@ __device__ inline bool split_lane(const Geo &g, int &s, int &f) {
   return s < g.sites;
 }
 
-// Element k of the array at `base` (wave-uniform).  OFF32 (every index of
-// the kernel below 2^29): the byte offset is formed in 32 bits, so the access
+// Element k of the array at `base` (wave-uniform).  OFF32 (every byte offset
+// of the kernel below 2^32): the byte offset is formed in 32 bits, so the access
 // takes the scalar base and a 32-bit lane offset instead of a 64-bit lane
 // address (one address register and no 64-bit arithmetic per access).
 template <bool OFF32, class T>
@@ -142,22 +142,34 @@ __device__ inline int nbr_site(int s, const NbrOffsets &o, int cx, int cy, int c
          (cz < 0 ? o.zm : (cz > 0 ? o.zp : 0));
 }
 
-// True when every population index of a lattice (19 sp) is below 2^29.
-inline bool split_off32(const Geo &g) { return 19 * g.sp < ((int64_t)1 << 29); }
+// Whether the byte offsets of a component's populations (FP64), or of both
+// components' (shifted storage, `elem` bytes a value), stay below 2^32.
+inline bool split_off32(const Geo &g) { return 19 * 8 * g.sp < ((int64_t)1 << 32); }
+inline bool shift_off32(const Geo &g, int elem) { return 38 * elem * g.sp < ((int64_t)1 << 32); }
+
+// tile_elem<19> of a site; OFF32: in 32 bits, with a 24-bit product (site
+// indices are below 2^30).
+template <bool OFF32>
+__device__ inline auto tile_off(int s) {
+  if constexpr (OFF32)
+    return (uint32_t)s + __umul24((uint32_t)s >> 6, 64u * 18u);
+  else
+    return tile_elem<19>(s);
+}
 
 // The 19 streamed populations of component f (array Af) at site s = (x, y, z)
 // whose solid word is sw (pull with bounce-back, src/dlbc/lb/advection.d:61-89).
-// Each load takes a wave-uniform base, array min(i, bounce(i)) of Af, and a
-// lane offset below 8 sp (bounce partners are at most 7 arrays apart).
+// Each load takes a wave-uniform base, population min(i, bounce(i)) of tile 0,
+// and a lane offset.
 template <bool SOLID, bool OFF32, class T>
 __device__ inline T pull_one(const T *__restrict__ Af, const Geo &g, int i, int s,
                              const NbrOffsets &o, uint32_t sw) {
   using L = D3Q19;
   const int src = nbr_site(s, o, -L::c[i][0], -L::c[i][1], -L::c[i][2]);
-  if (!SOLID) return at<OFF32>(Af + (int64_t)i * g.sp, src);
+  if (!SOLID) return at<OFF32>(Af + 64 * i, tile_off<OFF32>(src));
   const int b = L::bounce[i], mc = i < b ? i : b;
   const bool bb = (sw >> b) & 1u;
-  return at<OFF32>(Af + (int64_t)mc * g.sp, (int64_t)((bb ? b : i) - mc) * g.sp + (bb ? s : src));
+  return at<OFF32>(Af + 64 * mc, 64 * ((bb ? b : i) - mc) + tile_off<OFF32>(bb ? s : src));
 }
 
 template <bool SOLID, bool OFF32>
@@ -490,7 +502,7 @@ __global__ void __launch_bounds__(kSplitThreads)
   double *__restrict__ Bf = B + (int64_t)f * 19 * g.sp;
   collide_d3q19_streamed(f, n, rho, total, F, wv, p, [&](int i, double v) {
     __builtin_nontemporal_store(solid_site ? n[L::bounce[i]] : v,
-                                elem<OFF32>(Bf + (int64_t)i * g.sp, s));
+                                elem<OFF32>(Bf + 64 * i, tile_off<OFF32>(s)));
   });
 }
 
@@ -502,8 +514,8 @@ __global__ void __launch_bounds__(kSplitThreads)
 
 // Both components' streamed populations at site s (pull with bounce-back,
 // src/dlbc/lb/advection.d:61-89): one 8-byte (FP32) or 4-byte (FP16) load
-// per population and lane, from a wave-uniform base, array min(i, bounce(i)),
-// at a lane offset below 16 sp elements.
+// per population and lane, from a wave-uniform base, population
+// min(i, bounce(i)) of tile 0, at a lane offset.
 template <class Store, bool SOLID, bool OFF32>
 __device__ inline void ssplit_pull(const Store *__restrict__ A, const Geo &g, int s,
                                    const NbrOffsets &o, uint32_t sw, float (&n0)[19],
@@ -514,12 +526,11 @@ __device__ inline void ssplit_pull(const Store *__restrict__ A, const Geo &g, in
     const int src = nbr_site(s, o, -L::c[i][0], -L::c[i][1], -L::c[i][2]);
     const Store *p;
     if (!SOLID) {
-      p = elem<OFF32>(A + 2 * (int64_t)i * g.sp, 2 * (int64_t)src);
+      p = elem<OFF32>(A + 128 * i, 2 * tile_off<OFF32>(src));
     } else {
       const int b = L::bounce[i], mc = i < b ? i : b;
       const bool bb = (sw >> b) & 1u;
-      p = elem<OFF32>(A + 2 * (int64_t)mc * g.sp,
-                      2 * ((int64_t)((bb ? b : i) - mc) * g.sp + (bb ? s : src)));
+      p = elem<OFF32>(A + 128 * mc, 128 * ((bb ? b : i) - mc) + 2 * tile_off<OFF32>(bb ? s : src));
     }
     pair_load(p, n0[i], n1[i]);
   }
@@ -607,7 +618,7 @@ __device__ inline void ssplit_collide_block(const Store *__restrict__ A, Store *
                 [&](int i, float v) { n0[i] = solid_site ? n0[i] : v; });
   shifted_relax(n1, rho1, rho0, j1, j0, F1, p, pl1, [&](int i, float v) {
     const int b = L::bounce[i];
-    pair_store_nt<Store>(elem<OFF32>(B + 2 * (int64_t)i * g.sp, 2 * (int64_t)s),
+    pair_store_nt<Store>(elem<OFF32>(B + 128 * i, 2 * tile_off<OFF32>(s)),
                          solid_site ? n0[b] : n0[i], solid_site ? n1[b] : v);
   });
 }
@@ -668,7 +679,7 @@ inline void launch_ssplit_d3q19(const void *A, void *B, const uint32_t *nbw, flo
                                 int pass) {
   const Store *a = static_cast<const Store *>(A);
   Store *b = static_cast<Store *>(B);
-  if (split_off32(g))
+  if (shift_off32(g, sizeof(Store)))
     launch_ssplit_impl<Store, true>(a, b, nbw, P, g, p, stream, pass);
   else
     launch_ssplit_impl<Store, false>(a, b, nbw, P, g, p, stream, pass);
