@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -42,6 +43,13 @@ struct dlbc_gpu_ctx {
   float *P = nullptr;                       // shifted storage: psi in FP32 (split schedule)
   uint8_t *mask = nullptr;
   uint32_t *nbw = nullptr;  // solid-neighbour words (bit i: x + c_i solid)
+  // split schedule with both passes in one launch (split_one_launch): what its
+  // workgroups do, and the flags of the psi blocks (two sets in turn)
+  int32_t *order = nullptr;
+  int norder = 0;
+  uint8_t *psi_flags = nullptr;
+  int nflag = 0, psi_set = 0, psi_polls = kPsiPolls;
+  bool one_launch_off = false;  // no memory for them
   int has_solid = 0;
   bool params_set = false, pops_uploaded[kMaxC] = {false, false, false, false};
   bool solid_rho_dirty = true;
@@ -538,32 +546,103 @@ struct MarchStep {
   }
 };
 
+int effective_schedule(const dlbc_gpu_ctx *c) {
+  if (c->schedule != DLBC_SCHED_AUTO) return c->schedule;
+  // shifted storage: the split kernels (256^3 channel: FP32 1.25 against 2.40 ms,
+  // FP16 0.84 against 2.0); the tiled kernel (FUSED) remains selectable
+  if (c->storage != DLBC_STORAGE_F64) return DLBC_SCHED_SPLIT;
+  // D3Q19 two-component FP64: the lane-per-component two-pass kernels are the
+  // fastest measured schedule (256^3 channel: 2.57 ms/step vs 4.20 ms fused)
+  if (c->d == 3 && c->C == 2) return DLBC_SCHED_SPLIT;
+  return DLBC_SCHED_TWO_PASS;
+}
+
+// Sites per block of the split schedule.
+int split_sites(const dlbc_gpu_ctx *c) {
+  return c->storage == DLBC_STORAGE_F64 ? kSplitThreads / 2 : kShiftSites;
+}
+
+// Whether a Shan-Chen step of the split schedule is one launch.  us per step,
+// two launches against one: FP64 48^3 22 / 34, 64^3 42.6 / 42.5, 72^3 63.5 /
+// 61.3, 96^3 148 / 135, 256^3 2960 / 2385; FP32 80^3 42 / 48, 96^3 70 / 73,
+// 190x151x117 with solids 292 / 276, 256^3 1390 / 1157; FP16 without solids
+// 128^3 91 / 90, 256^3 719 / 680, 384^3 2570 / 2330.  FP16 with solids, whose
+// collide is bound by its instructions and whose psi then runs at the collide's
+// four waves per SIMD, 836 / 943 at 256^3: two launches.
+bool split_one_launch(const dlbc_gpu_ctx *c) {
+  if (c->d != 3 || c->C != 2 || !c->p.sc || c->geo.order_chunk != 0 || c->one_launch_off)
+    return false;
+  if (c->storage == DLBC_STORAGE_F16_SHIFT && c->has_solid) return false;
+  const int64_t blocks = c->storage == DLBC_STORAGE_F64 ? 2500 : 6000;
+  return c->geo.sites >= blocks * split_sites(c);
+}
+
+// The order and the flags of that launch, once per context.  Without the memory
+// for them the step stays at two launches.
+int split_ready(dlbc_gpu_ctx *c) {
+  if (c->order || effective_schedule(c) != DLBC_SCHED_SPLIT || !split_one_launch(c))
+    return DLBC_OK;
+  std::vector<int32_t> o;
+  try {
+    o = split_order(c->geo, split_sites(c));
+  } catch (const std::bad_alloc &) {
+    c->one_launch_off = true;
+    return DLBC_OK;
+  }
+  const int nflag = split_flags(blocks_for(c->geo.sites, split_sites(c)));
+  const size_t ob = sizeof(int32_t) * o.size();
+  int32_t *d = nullptr;
+  uint8_t *fl = nullptr;
+  if (hipMalloc(&d, ob) != hipSuccess || hipMalloc(&fl, 2 * (size_t)nflag) != hipSuccess) {
+    (void)hipGetLastError();
+    if (d) (void)hipFree(d);
+    c->one_launch_off = true;
+    return DLBC_OK;
+  }
+  hipError_t e = hipMemsetAsync(fl, 0, 2 * (size_t)nflag, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(d, o.data(), ob, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e != hipSuccess) {
+    (void)hipFree(d);
+    (void)hipFree(fl);
+    return fail(c, DLBC_ERR_HIP, "order of the split schedule: %s", hipGetErrorString(e));
+  }
+  c->order = d;
+  c->norder = 8 * (int)o.size();
+  c->psi_flags = fl;
+  c->nflag = nflag;
+  c->dev_bytes += (int64_t)(ob + 2 * (size_t)nflag);
+  return DLBC_OK;
+}
+
 // Lane-per-component two-pass schedule (D3Q19, two components, FP64).
 template <class L, int C>
 struct SplitStep {
   static int run(dlbc_gpu_ctx *c, Timer *tm, double *acc_ms) {
     (void)acc_ms;
     if constexpr (std::is_same<L, D3Q19>::value && C == 2) {
+      const SplitPlan q{c->order, c->psi_flags, c->nflag, c->psi_set, c->psi_polls};
       auto pass = [&](int k) {
+        tm->before();
         if (c->storage == DLBC_STORAGE_F64)
           launch_split_d3q19(static_cast<const double *>(c->popA),
-                             static_cast<double *>(c->popB), c->nbw, c->S, c->geo, c->p,
-                             c->stream, k);
+                             static_cast<double *>(c->popB), c->nbw, c->S, c->geo, c->p, q,
+                             c->norder, c->stream, k);
         else if (c->storage == DLBC_STORAGE_F32_SHIFT)
-          launch_ssplit_d3q19<float>(c->popA, c->popB, c->nbw, c->P, c->geo, c->sparams,
-                                     c->stream, k);
+          launch_ssplit_d3q19<float>(c->popA, c->popB, c->nbw, c->P, c->geo, c->sparams, q,
+                                     c->norder, c->stream, k);
         else
-          launch_ssplit_d3q19<__half>(c->popA, c->popB, c->nbw, c->P, c->geo, c->sparams,
-                                      c->stream, k);
-      };
-      if (c->p.sc) {
-        tm->before();
-        pass(0);
+          launch_ssplit_d3q19<__half>(c->popA, c->popB, c->nbw, c->P, c->geo, c->sparams, q,
+                                      c->norder, c->stream, k);
         tm->after();
+      };
+      if (split_one_launch(c)) {
+        pass(2);
+        c->psi_set ^= 1;
+      } else {
+        if (c->p.sc) pass(0);
+        pass(1);
       }
-      tm->before();
-      pass(1);
-      tm->after();
       std::swap(c->popA, c->popB);
       return DLBC_OK;
     } else {
@@ -607,17 +686,6 @@ int with_loader(dlbc_gpu_ctx *c, Fn fn) {
   return fn(D3Q19{}, ld);
 }
 
-int effective_schedule(const dlbc_gpu_ctx *c) {
-  if (c->schedule != DLBC_SCHED_AUTO) return c->schedule;
-  // shifted storage: the split pair (FP16 1.80 vs 1.94 ms on the 256^3 channel,
-  // FP32 even); the tiled kernel (FUSED) remains selectable
-  if (c->storage != DLBC_STORAGE_F64) return DLBC_SCHED_SPLIT;
-  // D3Q19 two-component FP64: the lane-per-component two-pass kernels are the
-  // fastest measured schedule (256^3 channel: 3.45 ms/step vs 4.51 ms fused)
-  if (c->d == 3 && c->C == 2) return DLBC_SCHED_SPLIT;
-  return DLBC_SCHED_TWO_PASS;
-}
-
 int prepare(dlbc_gpu_ctx *c) {
   if (!c->params_set) return fail(c, DLBC_ERR_STATE, "dlbc_gpu_set_params not called");
   for (int f = 0; f < c->C; ++f)
@@ -649,6 +717,7 @@ int step_once(dlbc_gpu_ctx *c, int sched, Timer *tm) {
 
 int do_steps(dlbc_gpu_ctx *c, int nsteps, Timer *tm) {
   int rc = prepare(c);
+  if (!rc) rc = split_ready(c);
   if (rc) return rc;
   const int sched = effective_schedule(c);
   for (int t = 0; t < nsteps; ++t) {
@@ -681,8 +750,11 @@ std::vector<unsigned char> graph_key(const dlbc_gpu_ctx *c, int sched) {
     const auto *b = static_cast<const unsigned char *>(p);
     k.insert(k.end(), b, b + n);
   };
-  const int ints[6] = {sched,         c->storage,   c->has_solid,
-                       c->target_blocks, c->march_rows, c->march_hold};
+  // the flag set and the buffer parity alternate together while the split
+  // schedule takes one launch per step
+  const int ints[8] = {sched,         c->storage,    c->has_solid, c->target_blocks,
+                       c->march_rows, c->march_hold, c->psi_set ^ (c->popA == c->bufX ? 0 : 1),
+                       c->psi_polls};
   put(ints, sizeof ints);
   put(&c->geo, sizeof c->geo);
   put(&c->p, sizeof c->p);
@@ -1346,6 +1418,7 @@ int dlbc_gpu_step_graph(dlbc_gpu_ctx *c, int nsteps) {
   if (!c || nsteps < 0) return DLBC_ERR_ARG;
   if (nsteps == 0) return DLBC_OK;
   int rc = prepare(c);
+  if (!rc) rc = split_ready(c);
   if (rc) return rc;
   const int sched = effective_schedule(c);
   if (c->storage != DLBC_STORAGE_F64 && sched == DLBC_SCHED_FUSED) {
@@ -1444,6 +1517,8 @@ const char *dlbc_gpu_kernel_name(const dlbc_gpu_ctx *c, int i) {
   if (sched == DLBC_SCHED_MARCH) return i == 0 ? "march_d3q19" : "";
   if (sched == DLBC_SCHED_SPLIT) {
     const bool sh = c->storage != DLBC_STORAGE_F64;
+    if (split_one_launch(c))
+      return i == 0 ? (sh ? "split_one_launch_shifted" : "split_one_launch") : "";
     if (c->p.sc)
       return i == 0 ? (sh ? "psi_split_shifted" : "psi_split")
                     : (i == 1 ? (sh ? "stream_force_collide_split_shifted"
@@ -1643,6 +1718,25 @@ int dlbc_gpu_eval_psi(dlbc_gpu_ctx *c, int psi_form, const double *x, double *y,
   return DLBC_OK;
 }
 
+int64_t dlbc_selftest_split_order(int nx, int ny, int nz, int block_sites) {
+  const int64_t sites = (int64_t)nx * ny * nz;
+  if (nx < 2 || ny < 2 || nz < 2 || sites > (1 << 26) || block_sites < 64) return -1;
+  Geo g;
+  g.nx = nx;
+  g.ny = ny;
+  g.nz = nz;
+  g.sites = (int)sites;
+  g.sp = (sites + 63) / 64 * 64;
+  geo_set_divisors(g);
+  return split_order_faults(g, block_sites, split_order(g, block_sites));
+}
+
+int dlbc_selftest_set_psi_polls(dlbc_gpu_ctx *c, int polls) {
+  if (!c || polls < 0 || polls > kPsiPolls) return DLBC_ERR_ARG;
+  c->psi_polls = polls;
+  return DLBC_OK;
+}
+
 int64_t dlbc_selftest_site_division(int64_t n, uint64_t seed) {
   uint64_t st = seed * 0x9E3779B97F4A7C15ull + 7;
   auto next = [&]() {  // splitmix64
@@ -1685,6 +1779,8 @@ void dlbc_gpu_destroy(dlbc_gpu_ctx *c) {
   if (c->P) (void)hipFree(c->P);
   if (c->mask) (void)hipFree(c->mask);
   if (c->nbw) (void)hipFree(c->nbw);
+  if (c->order) (void)hipFree(c->order);
+  if (c->psi_flags) (void)hipFree(c->psi_flags);
   if (c->scratch) (void)hipFree(c->scratch);
   if (c->d_self) (void)hipFree(c->d_self);
   if (c->d_items) (void)hipFree(c->d_items);

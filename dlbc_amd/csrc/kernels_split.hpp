@@ -15,6 +15,9 @@
 //   pass 2: pull again, Shan-Chen force from psi in S, velocity shift,
 //           BGK collision
 //
+// Large lattices take both passes in one launch (SplitPlan below), small ones
+// in two.
+//
 // When a block's sites lie in one z-row (n_z a multiple of the block's
 // sites), pass 2 stages the nine psi rows around the block in LDS with
 // coalesced loads issued after the pulls, instead of gathering 19 scattered
@@ -30,6 +33,7 @@
 
 #include "kernels_fused.hpp"
 #include "kernels_shifted.hpp"
+#include "split_order.hpp"
 
 namespace dlbc {
 
@@ -52,8 +56,7 @@ inline int split_grid(int64_t sites, int threads = kSplitThreads) {
 // neighbouring in y then share an XCD and its L2, and in x too when a plane
 // is a whole number of turns (8 K blocks).  Blocks from g.order_main on (the
 // part of the grid short of a whole turn) keep site order.
-__device__ inline int split_block(const Geo &g) {
-  const int b = blockIdx.x;
+__device__ inline int split_block(const Geo &g, int b) {
   const int K = g.order_chunk;
   if (K <= 0 || b >= g.order_main) return b;
   const int j = b >> 3;
@@ -87,13 +90,86 @@ __device__ inline bool line_all_solid(bool solid_site) {
 // threadIdx.x >> 6 is uniform, but the compiler cannot tell).
 __device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Site and component of this lane (the component is uniform per wave); false
-// past the end of the lattice.
-__device__ inline bool split_lane(const Geo &g, int &s, int &f) {
-  const int w = uniform(threadIdx.x >> 6);
+// Site and component of this lane in wave w of block blk (the component is
+// uniform per wave); false past the end of the lattice.
+__device__ inline bool split_lane(const Geo &g, int blk, int w, int &s, int &f) {
   f = w & 1;
-  s = uniform(split_block(g) * (kSplitThreads / 2) + (w >> 1) * 64) + (threadIdx.x & 63);
+  s = uniform(blk * (kSplitThreads / 2) + (w >> 1) * 64) + (threadIdx.x & 63);
   return s < g.sites;
+}
+
+// ---- both passes in one launch -------------------------------------------------
+// Every block of sites is visited by a psi workgroup and later by a collide
+// workgroup, in the order of a table (split_order.hpp).  psi goes from one to
+// the other through S (P): written through the L2 of the XCD that made it, and
+// then a flag for its block.  A collide wave looks at the flags of the blocks
+// that it reads before it reads them; until then no line of theirs is in its
+// L2, and a line is written by one wave with one store, so that no line is read
+// half written.
+// A wave that finds no flags for too long computes that psi itself (the same
+// values): no wave waits for one that has not started.
+struct SplitPlan {
+  const int32_t *order;  // what each turn of eight workgroups does
+  uint8_t *flags;        // [2][nflag]: the psi of a block is written
+  int nflag;             // flags of a set: the blocks rounded up to 8
+  int set;               // the flags this launch sets; it clears the others
+  int polls;             // looks at the flags before a wave computes the psi itself
+};
+
+// Flags of one set for nb blocks.
+inline int split_flags(int nb) { return (nb + 7) / 8 * 8; }
+
+// Nonzero in some lane while the psi that a collide of block blk of a lattice
+// reads is not all flagged.  Lane group k takes the k-th interval of
+// split_needs, a lane eight flags at a time.  blk0: the lattice's first flag.
+__device__ inline uint64_t psi_missing(const SplitPlan &q, const Geo &g, int SB, int blk0, int blk) {
+  const uint64_t *w = reinterpret_cast<const uint64_t *>(q.flags + (int64_t)q.set * q.nflag);
+  const int lane = threadIdx.x & 63;
+  int lo, hi;
+  split_needs(g, SB, blk, lane >> 3, lo, hi);
+  lo += blk0;
+  hi += blk0;
+  uint64_t miss = 0;
+  if (lo <= hi)
+    for (int k = (lo >> 3) + (lane & 7); k <= (hi >> 3); k += 8) {
+      uint64_t need = 0x0101010101010101ull;
+      if (k == (lo >> 3)) need &= ~0ull << (8 * (lo & 7));
+      if (k == (hi >> 3)) need &= ~0ull >> (56 - 8 * (hi & 7));
+      miss |= need & ~__hip_atomic_load(w + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  return miss;
+}
+
+// SplitPlan::polls: some tens of milliseconds, where a wave that the order
+// serves waits a few microseconds.
+constexpr int kPsiPolls = 1 << 14;
+
+// Polls until psi_missing is zero in all lanes; false when that took too long.
+__device__ inline bool psi_wait(const SplitPlan &q, const Geo &g, int SB, int blk0, int blk) {
+  for (int t = 0; t < q.polls; ++t)
+    if (__all(psi_missing(q, g, SB, blk0, blk) == 0)) return true;
+  return false;
+}
+
+// A psi value that workgroups on other XCDs read during this launch.
+template <bool SHARED, class T>
+__device__ inline void psi_store(T *p, T v) {
+  if constexpr (SHARED)
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    *p = v;
+}
+
+// Flag a block once every wave of the workgroup has its psi out (and clear the
+// flag for the next launch).
+__device__ inline void psi_publish(const SplitPlan &q, int blk) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(q.flags + (int64_t)q.set * q.nflag + blk, (uint8_t)1, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(q.flags + (int64_t)(q.set ^ 1) * q.nflag + blk, (uint8_t)0,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 // Element k of the array at `base` (wave-uniform).  OFF32 (every byte offset
@@ -216,7 +292,7 @@ __device__ inline void lane_coords(int s, const Geo &g, int &x, int &y, int &z) 
 // the loads overlap the population pulls issued before; the caller's barrier
 // publishes the rows.
 template <int SB, int THREADS, bool OFF32, class T>
-__device__ inline void stage_psi_rows(const T *__restrict__ S, const Geo &g, int s0,
+__device__ inline void stage_psi_rows(const T *S, const Geo &g, int s0,
                                       T (*rows)[9][SB + 2]) {
   constexpr int VEC = 16 / (int)sizeof(T);  // values per 16-byte load
   typedef T Vec __attribute__((ext_vector_type(VEC)));
@@ -270,19 +346,28 @@ __device__ inline T staged_psi(const T (*rows)[9][SB + 2], int ff, int i, int k)
   return rows[ff][(L::c[i][0] + 1) * 3 + L::c[i][1] + 1][k + 1 + L::c[i][2]];
 }
 
-template <bool SOLID, bool OFF32>
-__global__ void __launch_bounds__(kSplitThreads)
-    k_split_psi(const double *__restrict__ A, const uint32_t *__restrict__ nbw,
-                double *__restrict__ S, Geo g, int psi_form) {
+// psi of wave w's sites and component of block blk.
+template <bool SOLID, bool OFF32, bool SHARED>
+__device__ inline void split_psi_wave(const double *__restrict__ A,
+                                      const uint32_t *__restrict__ nbw, double *S, const Geo &g,
+                                      int psi_form, int blk, int w) {
   int s, f;
-  if (!split_lane(g, s, f)) return;
+  if (!split_lane(g, blk, w, s, f)) return;
   const uint32_t sw = SOLID ? nbw[s] : 0u;
   if (sw >> 31) return;  // solid: S keeps the site's density
   int x, y, z;
   lane_coords(s, g, x, y, z);
   double n[19];
   split_pull<SOLID, OFF32>(A + (int64_t)f * 19 * g.sp, g, s, nbr_offsets(g, x, y, z), sw, n);
-  *elem<OFF32>(S + (int64_t)f * g.sp, s) = psi_of(psi_form, density<D3Q19>(n));
+  psi_store<SHARED>(elem<OFF32>(S + (int64_t)f * g.sp, s), psi_of(psi_form, density<D3Q19>(n)));
+}
+
+template <bool SOLID, bool OFF32>
+__global__ void __launch_bounds__(kSplitThreads)
+    k_split_psi(const double *__restrict__ A, const uint32_t *__restrict__ nbw,
+                double *__restrict__ S, Geo g, int psi_form) {
+  split_psi_wave<SOLID, OFF32, false>(A, nbw, S, g, psi_form, split_block(g, blockIdx.x),
+                                      uniform(threadIdx.x >> 6));
 }
 
 // addShanChenForcePsi (src/dlbc/lb/force.d:238-309) for two components whose
@@ -422,11 +507,12 @@ __device__ inline void collide_d3q19_streamed(int f, const double *n, double rho
 // STAGED (n_z a multiple of the block's sites): the psi rows come from LDS.
 // A template argument rather than a runtime test, so that the body holds one
 // psi source: with both, every psi read sat behind a branch and a full wait.
-template <bool SOLID, bool OFFDIAG, bool OFF32, bool STAGED>
+// ONE: both passes in one launch (SplitPlan q); else the second pass alone.
+template <bool SOLID, bool OFFDIAG, bool OFF32, bool STAGED, bool ONE>
 __global__ void __launch_bounds__(kSplitThreads)
     k_split_collide(const double *__restrict__ A, double *__restrict__ B,
-                    const uint32_t *__restrict__ nbw, const double *__restrict__ S, Geo g,
-                    StepParams p) {
+                    const uint32_t *__restrict__ nbw, double *S, Geo g, StepParams p,
+                    SplitPlan q) {
   using L = D3Q19;
   constexpr int C = 2;
   constexpr int SB = kSplitThreads / 2;
@@ -435,8 +521,35 @@ __global__ void __launch_bounds__(kSplitThreads)
   // psi rows of the block when it lies in one z-row
   __shared__ double rows[STAGED ? 2 : 1][9][SB + 2];
   constexpr bool staged = STAGED;
+  const int w = uniform(threadIdx.x >> 6);
+  int blk;
+  if constexpr (ONE) {
+    const int32_t turn = q.order[blockIdx.x >> 3];
+    if ((int)(blockIdx.x & 7) >= turn_count(turn)) return;
+    blk = turn_first(turn) + (blockIdx.x & 7);
+    const bool is_psi = !turn_collide(turn);
+    if (is_psi || !psi_wait(q, g, SB, 0, blk)) {
+      // the wave's part of the block's psi, or (not waited for any longer) all
+      // psi that this collide reads
+      for (int i = 0; i < (is_psi ? 1 : 8); ++i) {
+        int b = blk, b1 = blk;
+        if (!is_psi) split_needs(g, SB, blk, i, b, b1);
+        for (; b <= b1; ++b)
+          for (int v = is_psi ? w : 0; v <= (is_psi ? w : kSplitThreads / 64 - 1); ++v)
+            split_psi_wave<SOLID, OFF32, true>(A, nbw, S, g, p.psi_form, b, v);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (is_psi) {
+        psi_publish(q, blk);
+        return;
+      }
+    }
+    asm volatile("" ::: "memory");  // psi is read from here on
+  } else {
+    blk = split_block(g, blockIdx.x);
+  }
   int s, f;
-  const bool inside = split_lane(g, s, f);
+  const bool inside = split_lane(g, blk, w, s, f);
   const int k = ((threadIdx.x >> 7) << 6) | (threadIdx.x & 63);  // site within the block
   const uint32_t sw = !inside ? (1u << 31) : (SOLID ? nbw[s] : 0u);
   NbrOffsets o{};
@@ -459,7 +572,7 @@ __global__ void __launch_bounds__(kSplitThreads)
     split_pull<SOLID, OFF32>(A + (int64_t)f * 19 * g.sp, g, s, o, solid_site ? 0x7ffffu : sw,
                              n);
   }
-  if (staged) stage_psi_rows<SB, kSplitThreads, OFF32>(S, g, split_block(g) * SB, rows);
+  if (staged) stage_psi_rows<SB, kSplitThreads, OFF32>(S, g, blk * SB, rows);
   if (active) {
     rho = density<L>(n);
     if (bdist2) first_moment<L>(n, mom);
@@ -537,18 +650,18 @@ __device__ inline void ssplit_pull(const Store *__restrict__ A, const Geo &g, in
 }
 
 // The sites of block blk of a lattice (kShiftSites from blk * kShiftSites),
-// one per lane.
-__device__ inline int shift_site(int blk) {
-  return uniform(blk * kShiftSites + (threadIdx.x & ~63)) + (threadIdx.x & 63);
+// one per lane of its waves w.
+__device__ inline int shift_site(int blk, int w) {
+  return uniform(blk * kShiftSites + 64 * w) + (threadIdx.x & 63);
 }
 
-// Pass 1 for block blk of a lattice: psi of both components into P.
-template <class Store, bool SOLID, bool OFF32>
-__device__ inline void ssplit_psi_block(const Store *__restrict__ A,
-                                        const uint32_t *__restrict__ nbw,
-                                        float *__restrict__ P, const Geo &g,
-                                        const ShiftParams &p, int blk) {
-  const int s = shift_site(blk);
+// Pass 1 for the sites of wave w of block blk of a lattice: psi of both
+// components into P.
+template <class Store, bool SOLID, bool OFF32, bool SHARED = false>
+__device__ inline void ssplit_psi_wave(const Store *__restrict__ A,
+                                       const uint32_t *__restrict__ nbw, float *P, const Geo &g,
+                                       const ShiftParams &p, int blk, int w) {
+  const int s = shift_site(blk, w);
   if (s >= g.sites) return;
   const uint32_t sw = SOLID ? nbw[s] : 0u;
   if (sw >> 31) return;  // solid: psi is not read there
@@ -556,8 +669,42 @@ __device__ inline void ssplit_psi_block(const Store *__restrict__ A,
   lane_coords(s, g, x, y, z);
   float n0[19], n1[19];
   ssplit_pull<Store, SOLID, OFF32>(A, g, s, nbr_offsets(g, x, y, z), sw, n0, n1);
-  *elem<OFF32>(P, s) = psi_f(p.psi_form, p.rho0[0] + shifted_drho(n0));
-  *elem<OFF32>(P + g.sp, s) = psi_f(p.psi_form, p.rho0[1] + shifted_drho(n1));
+  psi_store<SHARED>(elem<OFF32>(P, s), psi_f(p.psi_form, p.rho0[0] + shifted_drho(n0)));
+  psi_store<SHARED>(elem<OFF32>(P + g.sp, s), psi_f(p.psi_form, p.rho0[1] + shifted_drho(n1)));
+}
+
+// The start of a workgroup of a one-launch step: its psi (then false: nothing is
+// left to do), or the wait of a collide workgroup (true).  blk0: the lattice's
+// first block in q.
+template <class Store, bool SOLID, bool OFF32>
+__device__ inline bool shift_one_launch(const Store *__restrict__ A,
+                                        const uint32_t *__restrict__ nbw, float *P, const Geo &g,
+                                        const ShiftParams &p, const SplitPlan &q, int blk0,
+                                        int blk, bool collide) {
+  const int w = uniform(threadIdx.x >> 6);
+  if (!collide || !psi_wait(q, g, kShiftSites, blk0, blk)) {
+    for (int i = 0; i < (collide ? 8 : 1); ++i) {
+      int b = blk, b1 = blk;
+      if (collide) split_needs(g, kShiftSites, blk, i, b, b1);
+      for (; b <= b1; ++b)
+        for (int v = collide ? 0 : w; v <= (collide ? kShiftThreads / 64 - 1 : w); ++v)
+          ssplit_psi_wave<Store, SOLID, OFF32, true>(A, nbw, P, g, p, b, v);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (!collide) {
+      psi_publish(q, blk0 + blk);
+      return false;
+    }
+  }
+  asm volatile("" ::: "memory");  // psi is read from here on
+  return true;
+}
+
+template <class Store, bool SOLID, bool OFF32>
+__device__ inline void ssplit_psi_block(const Store *__restrict__ A,
+                                        const uint32_t *__restrict__ nbw, float *P, const Geo &g,
+                                        const ShiftParams &p, int blk) {
+  ssplit_psi_wave<Store, SOLID, OFF32>(A, nbw, P, g, p, blk, uniform(threadIdx.x >> 6));
 }
 
 // Pass 2 for block blk of a lattice; rows: LDS for the block's psi rows when
@@ -569,14 +716,13 @@ __device__ inline void ssplit_psi_block(const Store *__restrict__ A,
 // components with one access.
 template <class Store, bool SOLID, bool OFF32, bool STAGED = false>
 __device__ inline void ssplit_collide_block(const Store *__restrict__ A, Store *__restrict__ B,
-                                            const uint32_t *__restrict__ nbw,
-                                            const float *__restrict__ P, const Geo &g,
-                                            const ShiftParams &p, int blk,
+                                            const uint32_t *__restrict__ nbw, float *P,
+                                            const Geo &g, const ShiftParams &p, int blk,
                                             float (*rows)[9][kShiftSites + 2]) {
   using L = D3Q19;
   constexpr int SB = kShiftSites;
   constexpr bool staged = STAGED;
-  const int s = shift_site(blk);
+  const int s = shift_site(blk, uniform(threadIdx.x >> 6));
   const int k = threadIdx.x;  // site within the block
   const uint32_t sw = s >= g.sites ? (1u << 31) : (SOLID ? nbw[s] : 0u);
   NbrOffsets o{};
@@ -627,90 +773,110 @@ template <class Store, bool SOLID, bool OFF32>
 __global__ void __launch_bounds__(kShiftThreads)
     k_ssplit_psi(const Store *__restrict__ A, const uint32_t *__restrict__ nbw,
                  float *__restrict__ P, Geo g, ShiftParams p) {
-  ssplit_psi_block<Store, SOLID, OFF32>(A, nbw, P, g, p, split_block(g));
+  ssplit_psi_block<Store, SOLID, OFF32>(A, nbw, P, g, p, split_block(g, blockIdx.x));
 }
 
 // At most 128 VGPRs: four waves per SIMD.
-template <class Store, bool SOLID, bool OFF32, bool STAGED>
+template <class Store, bool SOLID, bool OFF32, bool STAGED, bool ONE>
 __global__ void __launch_bounds__(kShiftThreads) __attribute__((amdgpu_waves_per_eu(4)))
     k_ssplit_collide(const Store *__restrict__ A, Store *__restrict__ B,
-                     const uint32_t *__restrict__ nbw, const float *__restrict__ P, Geo g,
-                     ShiftParams p) {
+                     const uint32_t *__restrict__ nbw, float *P, Geo g, ShiftParams p,
+                     SplitPlan q) {
   __shared__ float rows[STAGED ? 2 : 1][9][kShiftSites + 2];
-  ssplit_collide_block<Store, SOLID, OFF32, STAGED>(A, B, nbw, P, g, p, split_block(g), rows);
+  int blk;
+  if constexpr (ONE) {
+    const int32_t turn = q.order[blockIdx.x >> 3];
+    if ((int)(blockIdx.x & 7) >= turn_count(turn)) return;
+    blk = turn_first(turn) + (blockIdx.x & 7);
+    if (!shift_one_launch<Store, SOLID, OFF32>(A, nbw, P, g, p, q, 0, blk, turn_collide(turn)))
+      return;
+  } else {
+    blk = split_block(g, blockIdx.x);
+  }
+  ssplit_collide_block<Store, SOLID, OFF32, STAGED>(A, B, nbw, P, g, p, blk, rows);
 }
 
 // Blocks of kShiftSites sites over a lattice.
 inline int shift_grid(int64_t sites) { return (int)((sites + kShiftSites - 1) / kShiftSites); }
 
+template <class Store, bool OFF32, bool STAGED, bool ONE>
+inline void launch_ssplit_collide(const Store *a, Store *b, const uint32_t *nbw, float *P,
+                                  const Geo &g, const ShiftParams &p, const SplitPlan &q, int nb,
+                                  hipStream_t stream) {
+  const dim3 grid(nb), block(kShiftThreads);
+  if (p.has_solid)
+    hipLaunchKernelGGL((k_ssplit_collide<Store, true, OFF32, STAGED, ONE>), grid, block, 0,
+                       stream, a, b, nbw, P, g, p, q);
+  else
+    hipLaunchKernelGGL((k_ssplit_collide<Store, false, OFF32, STAGED, ONE>), grid, block, 0,
+                       stream, a, b, nbw, P, g, p, q);
+}
+
+// pass 0: psi, 1: collide, 2: both in one launch of `norder` workgroups.
 template <class Store, bool OFF32>
 inline void launch_ssplit_impl(const Store *a, Store *b, const uint32_t *nbw, float *P,
-                               const Geo &g, const ShiftParams &p, hipStream_t stream,
-                               int pass) {
+                               const Geo &g, const ShiftParams &p, const SplitPlan &q, int norder,
+                               hipStream_t stream, int pass) {
   const int nb = shift_grid(g.sites);
   const dim3 grid(nb), block(kShiftThreads);
-  if (pass == 0) {
-    if (p.has_solid)
-      hipLaunchKernelGGL((k_ssplit_psi<Store, true, OFF32>), grid, block, 0, stream, a, nbw, P,
-                         g, p);
-    else
-      hipLaunchKernelGGL((k_ssplit_psi<Store, false, OFF32>), grid, block, 0, stream, a, nbw, P,
-                         g, p);
-  } else {
-    const bool staged = g.nz % kShiftSites == 0;
-    if (p.has_solid && staged)
-      hipLaunchKernelGGL((k_ssplit_collide<Store, true, OFF32, true>), grid, block, 0, stream, a,
-                         b, nbw, P, g, p);
-    else if (p.has_solid)
-      hipLaunchKernelGGL((k_ssplit_collide<Store, true, OFF32, false>), grid, block, 0, stream,
-                         a, b, nbw, P, g, p);
-    else if (staged)
-      hipLaunchKernelGGL((k_ssplit_collide<Store, false, OFF32, true>), grid, block, 0, stream,
-                         a, b, nbw, P, g, p);
-    else
-      hipLaunchKernelGGL((k_ssplit_collide<Store, false, OFF32, false>), grid, block, 0, stream,
-                         a, b, nbw, P, g, p);
-  }
+  const bool staged = g.nz % kShiftSites == 0;
+  if (pass == 0 && p.has_solid)
+    hipLaunchKernelGGL((k_ssplit_psi<Store, true, OFF32>), grid, block, 0, stream, a, nbw, P, g,
+                       p);
+  else if (pass == 0)
+    hipLaunchKernelGGL((k_ssplit_psi<Store, false, OFF32>), grid, block, 0, stream, a, nbw, P, g,
+                       p);
+  else if (pass == 2 && staged)
+    launch_ssplit_collide<Store, OFF32, true, true>(a, b, nbw, P, g, p, q, norder, stream);
+  else if (pass == 2)
+    launch_ssplit_collide<Store, OFF32, false, true>(a, b, nbw, P, g, p, q, norder, stream);
+  else if (staged)
+    launch_ssplit_collide<Store, OFF32, true, false>(a, b, nbw, P, g, p, q, nb, stream);
+  else
+    launch_ssplit_collide<Store, OFF32, false, false>(a, b, nbw, P, g, p, q, nb, stream);
 }
 
 template <class Store>
 inline void launch_ssplit_d3q19(const void *A, void *B, const uint32_t *nbw, float *P,
-                                const Geo &g, const ShiftParams &p, hipStream_t stream,
-                                int pass) {
+                                const Geo &g, const ShiftParams &p, const SplitPlan &q,
+                                int norder, hipStream_t stream, int pass) {
   const Store *a = static_cast<const Store *>(A);
   Store *b = static_cast<Store *>(B);
   if (shift_off32(g, sizeof(Store)))
-    launch_ssplit_impl<Store, true>(a, b, nbw, P, g, p, stream, pass);
+    launch_ssplit_impl<Store, true>(a, b, nbw, P, g, p, q, norder, stream, pass);
   else
-    launch_ssplit_impl<Store, false>(a, b, nbw, P, g, p, stream, pass);
+    launch_ssplit_impl<Store, false>(a, b, nbw, P, g, p, q, norder, stream, pass);
 }
 
-template <bool OFF32, bool STAGED>
-inline void launch_split_collide(const double *A, double *B, const uint32_t *nbw,
-                                 const double *S, const Geo &g, const StepParams &p,
+template <bool OFF32, bool STAGED, bool ONE>
+inline void launch_split_collide(const double *A, double *B, const uint32_t *nbw, double *S,
+                                 const Geo &g, const StepParams &p, const SplitPlan &q, int nb,
                                  hipStream_t stream, bool solid, bool offdiag) {
-  const dim3 grid(split_grid(g.sites)), block(kSplitThreads);
+  const dim3 grid(nb), block(kSplitThreads);
   if (solid && offdiag)
-    hipLaunchKernelGGL((k_split_collide<true, true, OFF32, STAGED>), grid, block, 0, stream, A,
-                       B, nbw, S, g, p);
+    hipLaunchKernelGGL((k_split_collide<true, true, OFF32, STAGED, ONE>), grid, block, 0, stream,
+                       A, B, nbw, S, g, p, q);
   else if (solid)
-    hipLaunchKernelGGL((k_split_collide<true, false, OFF32, STAGED>), grid, block, 0, stream, A,
-                       B, nbw, S, g, p);
+    hipLaunchKernelGGL((k_split_collide<true, false, OFF32, STAGED, ONE>), grid, block, 0, stream,
+                       A, B, nbw, S, g, p, q);
   else if (offdiag)
-    hipLaunchKernelGGL((k_split_collide<false, true, OFF32, STAGED>), grid, block, 0, stream, A,
-                       B, nbw, S, g, p);
+    hipLaunchKernelGGL((k_split_collide<false, true, OFF32, STAGED, ONE>), grid, block, 0, stream,
+                       A, B, nbw, S, g, p, q);
   else
-    hipLaunchKernelGGL((k_split_collide<false, false, OFF32, STAGED>), grid, block, 0, stream,
-                       A, B, nbw, S, g, p);
+    hipLaunchKernelGGL((k_split_collide<false, false, OFF32, STAGED, ONE>), grid, block, 0, stream,
+                       A, B, nbw, S, g, p, q);
 }
 
+// pass 0: psi, 1: collide, 2: both in one launch of `norder` workgroups.
 template <bool OFF32>
 inline void launch_split_impl(const double *A, double *B, const uint32_t *nbw, double *S,
-                              const Geo &g, const StepParams &p, hipStream_t stream, int pass) {
+                              const Geo &g, const StepParams &p, const SplitPlan &q, int norder,
+                              hipStream_t stream, int pass) {
   const int nb = split_grid(g.sites);
   const dim3 grid(nb), block(kSplitThreads);
+  const bool solid = p.has_solid != 0;
   if (pass == 0) {
-    if (p.has_solid)
+    if (solid)
       hipLaunchKernelGGL((k_split_psi<true, OFF32>), grid, block, 0, stream, A, nbw, S, g,
                          p.psi_form);
     else
@@ -719,19 +885,25 @@ inline void launch_split_impl(const double *A, double *B, const uint32_t *nbw, d
     return;
   }
   const bool offdiag = p.gcc[0][0] == 0.0 && p.gcc[1][1] == 0.0;
-  if (g.nz % (kSplitThreads / 2) == 0)
-    launch_split_collide<OFF32, true>(A, B, nbw, S, g, p, stream, p.has_solid != 0, offdiag);
+  const bool staged = g.nz % (kSplitThreads / 2) == 0;
+  if (pass == 2 && staged)
+    launch_split_collide<OFF32, true, true>(A, B, nbw, S, g, p, q, norder, stream, solid, offdiag);
+  else if (pass == 2)
+    launch_split_collide<OFF32, false, true>(A, B, nbw, S, g, p, q, norder, stream, solid,
+                                             offdiag);
+  else if (staged)
+    launch_split_collide<OFF32, true, false>(A, B, nbw, S, g, p, q, nb, stream, solid, offdiag);
   else
-    launch_split_collide<OFF32, false>(A, B, nbw, S, g, p, stream, p.has_solid != 0, offdiag);
+    launch_split_collide<OFF32, false, false>(A, B, nbw, S, g, p, q, nb, stream, solid, offdiag);
 }
 
 inline void launch_split_d3q19(const double *A, double *B, const uint32_t *nbw, double *S,
-                               const Geo &g, const StepParams &p, hipStream_t stream,
-                               int pass) {
+                               const Geo &g, const StepParams &p, const SplitPlan &q, int norder,
+                               hipStream_t stream, int pass) {
   if (split_off32(g))
-    launch_split_impl<true>(A, B, nbw, S, g, p, stream, pass);
+    launch_split_impl<true>(A, B, nbw, S, g, p, q, norder, stream, pass);
   else
-    launch_split_impl<false>(A, B, nbw, S, g, p, stream, pass);
+    launch_split_impl<false>(A, B, nbw, S, g, p, q, norder, stream, pass);
 }
 
 }  // namespace dlbc

@@ -5,8 +5,8 @@
 // later by a collide workgroup, which reads the psi of its neighbour sites.
 // The order keeps the two visits close, so that the second pull of the
 // populations finds what the first one left in the memory-side cache (256 MB),
-// and far enough apart that a collide workgroup does not wait: a psi workgroup
-// is `kOrderAhead` blocks ahead of where the next collide workgroup needs it.
+// and far enough apart that a collide workgroup does not wait: psi is
+// `kOrderAhead` blocks ahead of where the next collide workgroup needs it.
 //
 // A large plane is cut into strips of rows, and a strip is marched along x
 // before the next one: the distance between the two visits is then about one
@@ -14,8 +14,8 @@
 // few rows ahead of the collide strips (the first also holds the last row, its
 // periodic neighbour), so that every psi is computed once.
 //
-// The order is one of speed alone: a collide workgroup checks the blocks that
-// it reads (split_needs) and could compute them itself.
+// The order is one of speed alone: a collide wave checks the flags of the
+// blocks that it reads (split_needs) and can compute them itself.
 #pragma once
 
 #include <algorithm>
@@ -26,10 +26,25 @@
 
 namespace dlbc {
 
-// Blocks of a strip's plane, and blocks that psi is ahead.
-constexpr int kOrderStrip = 128, kOrderAhead = 768;
+// Blocks of a strip's plane, blocks that psi is ahead, and turns of psi in a
+// row.  FP64, 256^3 without solids: 2440 us per step with strips of 128 blocks
+// and psi and collide turns one by one, 2385 with psi in rows of eight turns
+// (one by one, workgroups that did nothing at all in the psi turns' place
+// slowed the collide workgroups by a quarter).  Strips of 64, 256 and a whole
+// plane (512 blocks): 2510, 2500 and 2610.  Psi 512 blocks ahead: 2830 (collide
+// workgroups wait: some 1280 workgroups are resident), 768 to 1024: the same,
+// 1500: 2510.
+constexpr int kOrderStrip = 128, kOrderAhead = 1024, kOrderRow = 8;
 
-constexpr int32_t kOrderNone = -1;  // an empty place (turns of eight workgroups stay whole)
+// A turn: what eight consecutive workgroups do (workgroup b runs on XCD b % 8, so
+// every XCD gets both kinds in equal parts).  Workgroup j < turn_count takes
+// block turn_first + j, the others nothing.
+constexpr int32_t order_turn(int first, int count, bool collide) {
+  return first << 5 | count << 1 | (collide ? 1 : 0);
+}
+__host__ __device__ inline int turn_first(int32_t t) { return t >> 5; }
+__host__ __device__ inline int turn_count(int32_t t) { return t >> 1 & 15; }
+__host__ __device__ inline bool turn_collide(int32_t t) { return t & 1; }
 
 // The blocks whose psi a collide of block blk reads, as intervals [lo, hi] of
 // blocks (empty where lo > hi): number k of eight.  Planes xa - 1 .. xb + 1
@@ -75,99 +90,115 @@ __host__ __device__ inline void split_needs(const Geo &g, int SB, int blk, int k
   hi = (x * plane + r1 * g.nz + g.nz - 1) / SB;
 }
 
-// The places of a launch: 2 blk for the psi of block blk, 2 blk + 1 for its
-// collide, kOrderNone for nothing.  Workgroup b runs on XCD b % 8; each turn of
-// eight is of one kind, so that every XCD gets both in equal parts.  chunk > 0
-// (a caller's choice): all psi first, and turns of `chunk` consecutive blocks for
-// each XCD.
-inline std::vector<int32_t> split_order(const Geo &g, int SB, int chunk,
-                                        int strip = kOrderStrip, int ahead = kOrderAhead) {
+// The psi blocks and the collide blocks of a lattice in the order of their
+// visits, numbered from blk0, appended to psi and col; need: for every collide
+// the psi places it wants in front of it, counted in the whole of psi.
+inline void split_order_lists(const Geo &g, int SB, int blk0, std::vector<int32_t> &psi,
+                              std::vector<int32_t> &col, std::vector<int32_t> &need,
+                              int strip = kOrderStrip) {
   const int nb = (g.sites + SB - 1) / SB;
   const int64_t plane = (int64_t)g.ny * g.nz;
-  std::vector<int32_t> psi, col, out;
-  psi.reserve(nb);
-  col.reserve(nb);
+  const size_t psi0 = psi.size(), col0 = col.size();
   // first block that starts at or after site s
   auto first = [&](int64_t s) {
     return (int)std::min<int64_t>(nb, (std::max<int64_t>(s, 0) + SB - 1) / SB);
   };
   const int64_t wrap0 = plane - g.nz - SB + 1;  // blocks from here hold a plane's last row
-  if (chunk > 0) {
-    const int main = nb / (8 * chunk) * (8 * chunk);
-    for (int b = 0; b < nb; ++b) {
-      const int j = b >> 3;
-      psi.push_back(b >= main ? b : ((j / chunk) * 8 + (b & 7)) * chunk + j % chunk);
+  const int64_t pb = (plane + SB - 1) / SB;     // blocks of a plane
+  int ns = (int)std::max<int64_t>(1, (pb + strip / 2) / strip);
+  ns = std::min(ns, std::max(1, g.ny / 4));
+  const int H = (g.ny + ns - 1) / ns;  // rows of a strip
+  ns = (g.ny + H - 1) / H;
+  const int e = (SB + g.nz - 1) / g.nz + 1;  // rows that psi strips lie ahead
+  // the block that runs into the last plane, which the first collides read
+  const int64_t s_last = (int64_t)(g.nx - 1) * plane;
+  const int into = s_last % SB ? (int)(s_last / SB) : -1;
+  const int64_t into_at = into >= 0 ? (int64_t)into * SB % plane : 0;
+  for (int j = 0; j < ns; ++j) {
+    const bool last = j == ns - 1, wraps = j == 0 && !last;
+    const int y0 = j * H, y1 = last ? g.ny : (j + 1) * H;
+    auto edge = [&](int y) { return std::min<int64_t>((int64_t)(y + e) * g.nz, wrap0); };
+    // the psi strip's part of a plane; the first strip also takes the plane's end
+    const int64_t p0 = j == 0 ? 0 : edge(y0);
+    const int64_t p1 = !last ? edge(y1) : (j == 0 ? plane : wrap0);
+    if (into >= 0 && ((into_at >= p0 && into_at < p1) || (wraps && into_at >= wrap0)))
+      psi.push_back(blk0 + into);
+    auto put = [&](int lo, int hi) {
+      for (int b = lo; b < hi; ++b)
+        if (b != into) psi.push_back(blk0 + b);
+    };
+    for (int k = 0; k < g.nx; ++k) {  // from the last plane, which plane 0 reads
+      const int64_t base = (k == 0 ? g.nx - 1 : k - 1) * plane;
+      put(first(base + p0), first(base + p1));
+      if (wraps) put(std::max(first(base + p1), first(base + wrap0)), first(base + plane));
     }
-    col = psi;
-  } else {
-    const int64_t pb = (plane + SB - 1) / SB;  // blocks of a plane
-    int ns = (int)std::max<int64_t>(1, (pb + strip / 2) / strip);
-    ns = std::min(ns, std::max(1, g.ny / 4));
-    const int H = (g.ny + ns - 1) / ns;
-    ns = (g.ny + H - 1) / H;
-    const int e = (SB + g.nz - 1) / g.nz + 1;  // rows that psi strips lie ahead
-    // the block that runs into the last plane, which the first collides read
-    const int64_t s_last = (int64_t)(g.nx - 1) * plane;
-    const int into = s_last % SB ? (int)(s_last / SB) : -1;
-    const int64_t into_at = into >= 0 ? (int64_t)into * SB % plane : 0;
-    for (int j = 0; j < ns; ++j) {
-      const bool last = j == ns - 1, wraps = j == 0 && !last;
-      const int y0 = j * H, y1 = last ? g.ny : (j + 1) * H;
-      auto edge = [&](int y) { return std::min<int64_t>((int64_t)(y + e) * g.nz, wrap0); };
-      const int64_t p0 = j == 0 ? 0 : edge(y0), p1 = j == 0 && last ? plane
-                                                     : last         ? wrap0
-                                                                    : edge(y1);
-      if (into >= 0 && ((into_at >= p0 && into_at < p1) || (wraps && into_at >= wrap0)))
-        psi.push_back(into);
-      auto put = [&](int lo, int hi) {
-        for (int b = lo; b < hi; ++b)
-          if (b != into) psi.push_back(b);
-      };
-      for (int k = 0; k < g.nx; ++k) {
-        const int64_t base = (k == 0 ? g.nx - 1 : k - 1) * plane;
-        put(first(base + p0), first(base + p1));
-        if (wraps) put(std::max(first(base + p1), first(base + wrap0)), first(base + plane));
-      }
-      for (int x = 0; x < g.nx; ++x) {
-        const int64_t base = x * plane;
-        for (int b = first(base + (int64_t)y0 * g.nz);
-             b < first(base + (last ? plane : (int64_t)y1 * g.nz)); ++b)
-          col.push_back(b);
-      }
+    for (int x = 0; x < g.nx; ++x) {
+      const int64_t base = x * plane;
+      for (int b = first(base + (int64_t)y0 * g.nz);
+           b < first(base + (last ? plane : (int64_t)y1 * g.nz)); ++b)
+        col.push_back(blk0 + b);
     }
   }
-  // the psi places that a block's collide needs in front of it
   std::vector<int32_t> place(nb);
-  for (int k = 0; k < nb; ++k) place[psi[k]] = k;
-  auto need = [&](int blk) {
-    if (chunk > 0) return nb;
+  for (int k = 0; k < nb; ++k) place[psi[psi0 + k] - blk0] = k;
+  for (size_t c = col0; c < col.size(); ++c) {
     int n = 0;
     for (int k = 0; k < 8; ++k) {
       int lo, hi;
-      split_needs(g, SB, blk, k, lo, hi);
+      split_needs(g, SB, col[c] - blk0, k, lo, hi);
       if (lo > hi) continue;
-      if (k == 0 && hi == nb - 1 && lo == 0) return nb;
       // places rise with the block but for the blocks taken early: those of a
       // plane's end and the one that runs into the last plane
-      const bool end = (int64_t)hi * SB % plane >= wrap0;
-      for (int v = end ? lo : std::max(lo, hi - 1); v <= hi; ++v) n = std::max(n, place[v] + 1);
+      const bool all = lo == 0 && hi == nb - 1, end = (int64_t)hi * SB % plane >= wrap0;
+      if (all) n = nb;
+      for (int v = all ? hi + 1 : (end ? lo : std::max(lo, hi - 1)); v <= hi; ++v)
+        n = std::max(n, place[v] + 1);
     }
+    need.push_back((int32_t)psi0 + n);
+  }
+}
+
+// The turns of a launch over these lists: runs of consecutive blocks, psi in
+// front of every collide by `ahead` blocks.
+inline std::vector<int32_t> split_order_merge(const std::vector<int32_t> &psi,
+                                              const std::vector<int32_t> &col,
+                                              const std::vector<int32_t> &need,
+                                              int ahead = kOrderAhead) {
+  std::vector<int32_t> out;
+  out.reserve((psi.size() + col.size()) / 8 + (psi.size() + col.size()) / 64 + 32);
+  size_t pp = 0, cp = 0;
+  auto run = [](const std::vector<int32_t> &v, size_t p) {
+    int n = 1;
+    while (n < 8 && p + n < v.size() && v[p + n] == v[p] + n) ++n;
     return n;
   };
-  // psi in front of every collide place by `ahead`, in turns of eight
-  size_t pp = 0, cp = 0;
-  auto turn = [&](const std::vector<int32_t> &v, size_t &p, int kind) {
-    for (int k = 0; k < 8; ++k, ++p) out.push_back(p < v.size() ? 2 * v[p] + kind : kOrderNone);
-  };
-  out.reserve(2 * (size_t)nb + 32);
   while (cp < col.size()) {
+    const int c = run(col, cp);
     int n = 0;
-    for (size_t k = cp; k < std::min(cp + 8, col.size()); ++k) n = std::max(n, need(col[k]));
-    while (pp < psi.size() && pp < (size_t)n + ahead) turn(psi, pp, 0);
-    turn(col, cp, 1);
+    for (int k = 0; k < c; ++k) n = std::max(n, need[cp + k]);
+    const bool due = pp < (size_t)n + ahead;
+    while (due && pp < psi.size() && pp < (size_t)n + ahead + 8 * (kOrderRow - 1)) {
+      const int k = run(psi, pp);
+      out.push_back(order_turn(psi[pp], k, false));
+      pp += k;
+    }
+    out.push_back(order_turn(col[cp], c, true));
+    cp += c;
   }
-  while (pp < psi.size()) turn(psi, pp, 0);
+  while (pp < psi.size()) {
+    const int k = run(psi, pp);
+    out.push_back(order_turn(psi[pp], k, false));
+    pp += k;
+  }
   return out;
+}
+
+// The order of one lattice.
+inline std::vector<int32_t> split_order(const Geo &g, int SB, int strip = kOrderStrip,
+                                        int ahead = kOrderAhead) {
+  std::vector<int32_t> psi, col, need;
+  split_order_lists(g, SB, 0, psi, col, need, strip);
+  return split_order_merge(psi, col, need, ahead);
 }
 
 // What is wrong with an order: blocks that are not visited once by each kind,
@@ -178,15 +209,16 @@ inline int64_t split_order_faults(const Geo &g, int SB, const std::vector<int32_
   std::vector<int64_t> at[2];
   at[0].assign(nb, -1);
   at[1].assign(nb, -1);
-  int64_t bad = o.size() % 8 != 0;
-  for (size_t p = 0; p < o.size(); ++p) {
-    if (o[p] == kOrderNone) continue;
-    if (o[p] < 0 || o[p] >= 2 * nb || at[o[p] & 1][o[p] >> 1] != -1) {
-      ++bad;
-      continue;
+  int64_t bad = 0;
+  for (size_t p = 0; p < o.size(); ++p)
+    for (int j = 0; j < turn_count(o[p]); ++j) {
+      const int b = turn_first(o[p]) + j, k = turn_collide(o[p]) ? 1 : 0;
+      if (b < 0 || b >= nb || turn_count(o[p]) > 8 || at[k][b] != -1) {
+        ++bad;
+        continue;
+      }
+      at[k][b] = (int64_t)p;
     }
-    at[o[p] & 1][o[p] >> 1] = (int64_t)p;
-  }
   for (int b = 0; b < nb; ++b) {
     if (at[0][b] < 0 || at[1][b] < 0) {
       ++bad;

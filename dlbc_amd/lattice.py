@@ -88,6 +88,8 @@ def lib():
         "dlbc_gpu_last_error": (C.c_char_p, [vp]),
         "dlbc_selftest_division": (i64, [i64, C.c_uint64]),
         "dlbc_selftest_site_division": (i64, [i64, C.c_uint64]),
+        "dlbc_selftest_split_order": (i64, [i, i, i, i]),
+        "dlbc_selftest_set_psi_polls": (i, [vp, i]),
         "dlbc_gpu_destroy": (None, [vp]),
         "dlbc_gpu_device_bytes": (i64, [vp]),
         "dlbc_rng_seed": (None, [C.POINTER(_Rng), C.c_uint32]),

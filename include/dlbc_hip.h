@@ -228,6 +228,17 @@ int64_t dlbc_selftest_division(int64_t n, uint64_t seed);
  * no GPU needed; no counterpart in the reference. */
 int64_t dlbc_selftest_site_division(int64_t n, uint64_t seed);
 
+/* Test entries of the one-launch split schedule.  The faults of the order of
+ * its workgroups for an n_x x n_y x n_z lattice (blocks of block_sites sites):
+ * a block not visited once by each kind, a neighbour whose psi a collide would
+ * not wait for, psi that stands behind a collide that needs it.  0: none; -1:
+ * arguments out of range. */
+int64_t dlbc_selftest_split_order(int nx, int ny, int nz, int block_sites);
+
+/* How often a collide wave of this context looks for the psi it reads before it
+ * computes it itself (0: at once).  Results do not depend on it. */
+int dlbc_selftest_set_psi_polls(dlbc_gpu_ctx *ctx, int polls);
+
 const char *dlbc_gpu_last_error(const dlbc_gpu_ctx *ctx);
 void dlbc_gpu_destroy(dlbc_gpu_ctx *ctx);
 

@@ -1,0 +1,77 @@
+"""The split schedule's one-launch step (psi and collide workgroups in one
+launch, in the order of a table): the order on the CPU; on the GPU the same
+bits as the oracle and as two launches, at the smallest lattices that take it
+and with planes cut into strips."""
+import numpy as np
+import pytest
+
+
+@pytest.mark.parametrize("n", [(2, 2, 2), (2, 3, 4), (3, 3, 3), (5, 7, 9), (100, 4, 4), (1000, 2, 2),
+                               (4, 4, 1000), (64, 64, 64), (12, 10, 128), (6, 40, 256),
+                               (31, 97, 65), (17, 64, 512), (9, 260, 127), (9, 300, 301),
+                               (2, 5000, 7), (3, 700, 129), (7, 5, 3000), (4, 256, 256)])
+@pytest.mark.parametrize("sites", [128, 256])
+def test_order_visits_every_block_and_never_waits_for_a_later_one(n, sites):
+    import dlbc_amd as D
+    assert D.lib().dlbc_selftest_split_order(*n, sites) == 0
+
+
+def _params(n, form, solid):
+    rng = np.random.default_rng(sum(n))
+    p = dict(d=3, q=19, gn=list(n), components=2, tau=[1.0, 0.9], eqDistForm=form,
+             gcc=[[0.0, 3.6], [3.6, 0.0]], enableShanChen=True, psiForm="Exponential",
+             fluidInit=["EqDistPerturb"] * 2, fluidDensities=[[0.7], [0.6]],
+             fluidPerturb=[0.02, 0.02], randomReseed=[True] * 2, randomSeed=[5, 6])
+    if solid:
+        p["gwc"] = [0.1, -0.1]
+        p["maskArray"] = (rng.random(n) < 0.1).astype(np.int32)
+    return p
+
+
+def _same(a, b, what):
+    for f in range(2):
+        x, y = a.population(f), b.population(f)
+        assert np.array_equal(x.view(np.uint64), y.view(np.uint64)), (what, f)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [(70, 90, 61), (2, 1250, 131), (16, 200, 128), (15, 211, 131),
+                               (41, 3, 2620)], ids=str)
+@pytest.mark.parametrize("form,solid", [("BDist2", True), ("SecondOrder", False)])
+def test_f64_equals_oracle(n, form, solid):
+    import dlbc_amd as D
+    from oracle.oracle import Oracle
+    p = _params(n, form, solid)
+    g, o = D.Lattice.from_params(p, schedule="split"), Oracle.from_params(p)
+    g.step(3)
+    o.run(3)
+    _same(g, o, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage,n", [("f64", (15, 211, 131)), ("f32_shift", (70, 150, 149)),
+                                       ("f32_shift", (13, 470, 256)), ("f16_shift", (24, 256, 256))],
+                         ids=str)
+@pytest.mark.parametrize("solid", [True, False])
+def test_equals_two_launches(storage, n, solid):
+    """Any block order keeps two launches per step; both give the same bits,
+    also in turn, over odd step counts, from a graph and where no collide wave
+    waits for the psi it reads (each computes it)."""
+    import dlbc_amd as D
+    p = _params(n, "BDist2", solid)
+    a, b = (D.Lattice.from_params(p, storage=storage, schedule="split") for _ in range(2))
+    b.set_block_order(8)
+    for k in (3, 1, 4):
+        a.step(k)
+        b.step(k)
+    _same(a, b, "steps")
+    a.set_block_order(8)
+    a.step(1)
+    a.set_block_order(0)
+    a.step(33, graph=True)
+    b.step(34)
+    _same(a, b, "block order, then a graph")
+    a._check(D.lib().dlbc_selftest_set_psi_polls(a.h, 0), "polls")
+    a.step(1)
+    b.step(1)
+    _same(a, b, "no waiting")
