@@ -1808,12 +1808,18 @@ struct dlbc_batch {
   std::vector<BatchItem> h_items;
   std::vector<int> lat_first;  // first item of each lattice, and the total
   int ty = 8, chunk = 1 << 20, grid = 512;
-  int kernel = 0;  // tiled: 0 solid-capable, 1 without solids; 2: the split pair;
+  int kernel = 0;  // tiled: 0 solid-capable, 1 without solids; 2: the split kernels;
                    // 3: the split pair as one persistent (cooperative) launch
   int coop_grid = 0;     // workgroups of that launch (0: not yet queried)
   int coop_variant = -1;  // the kernel variant coop_grid was queried for
   int *d_first = nullptr;     // split: first 128-site block of each member, and the total
   std::vector<int> h_first;
+  // split pair in one launch: its turns (each with its lattice) and flags
+  int32_t *order = nullptr;
+  int norder = 0;
+  uint8_t *psi_flags = nullptr;
+  int nflag = 0, psi_set = 0;
+  bool one_launch_off = false;  // no memory for them
   bool items_dirty = true;
   hipGraphExec_t graph = nullptr;
   int graph_sig = -1;  // batch_launch_sig() when the graph was captured
@@ -1887,12 +1893,64 @@ bool batch_has_sc(const dlbc_batch *b, int l0, int l1) {
   return false;
 }
 
+// Whether the split pair of the whole batch is one launch (the rule of
+// split_one_launch).
+bool batch_one_launch(const dlbc_batch *b) {
+  if (b->one_launch_off || !batch_has_sc(b, 0, (int)b->ctx.size())) return false;
+  if (b->storage == DLBC_STORAGE_F16_SHIFT && batch_has_solid(b)) return false;
+  return b->h_first.back() >= 6000;
+}
+
 // The host state that picks kernels at launch beyond the configuration: any
-// member with solids (the tiled kernel's SOLID variant) and any with
-// Shan-Chen (the split schedule's psi pass).  A captured graph is only valid
-// for the value it was captured with.
+// member with solids (the kernels' SOLID variants) and any with Shan-Chen (the
+// split schedule's psi pass), one launch or two and the flags it starts with.
+// A captured graph is only valid for the value it was captured with.
 int batch_launch_sig(const dlbc_batch *b) {
-  return (batch_has_solid(b) ? 1 : 0) | (batch_has_sc(b, 0, (int)b->ctx.size()) ? 2 : 0);
+  return (batch_has_solid(b) ? 1 : 0) | (batch_has_sc(b, 0, (int)b->ctx.size()) ? 2 : 0) |
+         (batch_one_launch(b) ? 4 + 8 * b->psi_set : 0);
+}
+
+// The turns and flags of that launch, once per batch; without the memory for
+// them the batch stays at two launches.
+int batch_split_ready(dlbc_batch *b) {
+  if (b->order || b->kernel != 2 || !batch_one_launch(b)) return DLBC_OK;
+  std::vector<int32_t> turns;
+  try {
+    std::vector<int32_t> psi, col, need;
+    for (size_t l = 0; l < b->ctx.size(); ++l)
+      split_order_lists(b->ctx[l]->geo, kShiftSites, b->h_first[l], psi, col, need);
+    for (int32_t t : split_order_merge(psi, col, need, kOrderAhead, b->h_first)) {
+      const auto next = std::upper_bound(b->h_first.begin(), b->h_first.end(), turn_first(t));
+      turns.push_back(t);
+      turns.push_back((int32_t)(next - b->h_first.begin()) - 1);
+    }
+  } catch (const std::bad_alloc &) {
+    b->one_launch_off = true;
+    return DLBC_OK;
+  }
+  const int nflag = split_flags(b->h_first.back());
+  const size_t ob = sizeof(int32_t) * turns.size();
+  int32_t *d = nullptr;
+  uint8_t *fl = nullptr;
+  if (hipMalloc(&d, ob) != hipSuccess || hipMalloc(&fl, 2 * (size_t)nflag) != hipSuccess) {
+    (void)hipGetLastError();
+    if (d) (void)hipFree(d);
+    b->one_launch_off = true;
+    return DLBC_OK;
+  }
+  hipError_t e = hipMemsetAsync(fl, 0, 2 * (size_t)nflag, b->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(d, turns.data(), ob, hipMemcpyHostToDevice, b->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
+  if (e != hipSuccess) {
+    (void)hipFree(d);
+    (void)hipFree(fl);
+    return bfail(b, DLBC_ERR_HIP, "order of the split batch: %s", hipGetErrorString(e));
+  }
+  b->order = d;
+  b->norder = 4 * (int)turns.size();  // eight workgroups a turn
+  b->psi_flags = fl;
+  b->nflag = nflag;
+  return DLBC_OK;
 }
 
 // Make every member ready (solid densities, pending uploads done) and the
@@ -1920,6 +1978,8 @@ int batch_prepare(dlbc_batch *b) {
     b->h_lats = t;
     b->lats_valid = true;
   }
+  const int rs = batch_split_ready(b);
+  if (rs) return rs;
   if (b->graph && b->graph_sig != batch_launch_sig(b)) batch_drop_graph(b);
   if (b->items_dirty) return batch_build_items(b);
   return DLBC_OK;
@@ -1933,25 +1993,40 @@ bool batch_off32(const dlbc_batch *b) {
   return true;
 }
 
-// Split schedule over the members [l0, l1).
+// Split schedule over the members [l0, l1): two launches, or one for a whole
+// batch that batch_split_ready has made ready.
 int batch_launch_split(dlbc_batch *b, int l0, int l1, int parity) {
   const int nlat = (int)b->ctx.size();
   const int blk0 = b->h_first[l0], nblk = b->h_first[l1] - blk0;
   const bool psi = batch_has_sc(b, l0, l1);
-  const bool f32 = b->storage == DLBC_STORAGE_F32_SHIFT, o32 = batch_off32(b);
-  if (f32 && o32)
-    launch_batch_split<float, true>(b->d_lats, b->d_first, nlat, blk0, nblk, parity, psi,
-                                    b->stream);
-  else if (f32)
-    launch_batch_split<float, false>(b->d_lats, b->d_first, nlat, blk0, nblk, parity, psi,
-                                     b->stream);
-  else if (o32)
-    launch_batch_split<__half, true>(b->d_lats, b->d_first, nlat, blk0, nblk, parity, psi,
-                                     b->stream);
-  else
-    launch_batch_split<__half, false>(b->d_lats, b->d_first, nlat, blk0, nblk, parity, psi,
+  const bool one = l0 == 0 && l1 == nlat && b->order && batch_one_launch(b);
+  const SplitPlan q{b->order, b->psi_flags, b->nflag, b->psi_set, kPsiPolls};
+  auto go = [&](auto store, auto solid, auto o32) {
+    using Store = decltype(store);
+    constexpr bool S = decltype(solid)::value, O = decltype(o32)::value;
+    if (one)
+      launch_batch_one<Store, S, O>(b->d_lats, b->d_first, nlat, parity, q, b->norder, b->stream);
+    else
+      launch_batch_split<Store, S, O>(b->d_lats, b->d_first, nlat, blk0, nblk, parity, psi,
                                       b->stream);
+  };
+  auto with_store = [&](auto solid, auto o32) {
+    if (b->storage == DLBC_STORAGE_F32_SHIFT)
+      go(float{}, solid, o32);
+    else
+      go(__half{}, solid, o32);
+  };
+  const bool solid = batch_has_solid(b), o32 = batch_off32(b);
+  if (solid && o32)
+    with_store(std::true_type{}, std::true_type{});
+  else if (solid)
+    with_store(std::true_type{}, std::false_type{});
+  else if (o32)
+    with_store(std::false_type{}, std::true_type{});
+  else
+    with_store(std::false_type{}, std::false_type{});
   BHIPCHK(b, hipGetLastError());
+  if (one) b->psi_set ^= 1;
   return DLBC_OK;
 }
 
@@ -2157,8 +2232,10 @@ int dlbc_batch_autotune(dlbc_batch *b, int *out, double *best_ms) {
     ms_out = ms / 3.0;
     return DLBC_OK;
   };
-  for (int kn : {2, 3}) {  // the split pair, two launches or one: no tile or chunk to tune
+  for (int kn : {2, 3}) {  // the split pair: no tile or chunk to tune
     b->kernel = kn;
+    rc = batch_split_ready(b);
+    if (rc) return rc;
     double ms;
     rc = trial(0, b->grid, ms);
     if (rc) return rc;
@@ -2220,6 +2297,8 @@ void dlbc_batch_destroy(dlbc_batch *b) {
   if (b->d_lats) (void)hipFree(b->d_lats);
   if (b->d_items) (void)hipFree(b->d_items);
   if (b->d_first) (void)hipFree(b->d_first);
+  if (b->order) (void)hipFree(b->order);
+  if (b->psi_flags) (void)hipFree(b->psi_flags);
   if (b->done) (void)hipEventDestroy(b->done);
   if (b->e0) (void)hipEventDestroy(b->e0);
   if (b->e1) (void)hipEventDestroy(b->e1);

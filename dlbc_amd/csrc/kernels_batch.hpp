@@ -337,9 +337,10 @@ inline int launch_batch_d3q19(const BatchLattice *lats, const BatchItem *items, 
 }
 
 // ---- batches on the split schedule -------------------------------------------
-// Two launches per step over all members: pass 1 (psi) then pass 2 (collide).
+// One launch per step over all members in the order of a table (split_order.hpp),
+// or two launches: pass 1 (psi) then pass 2 (collide).
 // Block b of a launch belongs to the lattice l with first[l] <= blk0 + b <
-// first[l + 1] (first: the prefix sums of the members' 128-site block counts).
+// first[l + 1] (first: the prefix sums of the members' 256-site block counts).
 
 __device__ inline int batch_block_lattice(const int *__restrict__ first, int nlat, int b) {
   int lo = 0, hi = nlat;  // first[lo] <= b < first[hi]
@@ -353,7 +354,10 @@ __device__ inline int batch_block_lattice(const int *__restrict__ first, int nla
   return lo;
 }
 
-template <class Store, bool OFF32>
+// SOLID: some member has solid sites (one without has all-zero solid words and
+// takes the same arithmetic path).  Without, the collide takes 88 VGPRs instead
+// of 122: five waves per SIMD.
+template <class Store, bool SOLID, bool OFF32>
 __global__ void __launch_bounds__(kShiftThreads)
     k_batch_split_psi(const BatchLattice *__restrict__ lats, const int *__restrict__ first,
                       int nlat, int blk0, int blk1, int parity) {
@@ -361,34 +365,49 @@ __global__ void __launch_bounds__(kShiftThreads)
   if (b >= blk1) return;
   const int l = uniform(batch_block_lattice(first, nlat, b));
   ConstLattice &B = table_entry(lats, l);
-  const Store *A = static_cast<const Store *>(B.pop[parity]);
   const Geo g = B.g;
   const ShiftParams p = B.p;
   if (!p.sc) return;  // this member's collide pass reads no psi
-  if (p.has_solid)
-    ssplit_psi_block<Store, true, OFF32>(A, B.nbw, B.P, g, p, b - first[l]);
-  else
-    ssplit_psi_block<Store, false, OFF32>(A, B.nbw, B.P, g, p, b - first[l]);
+  ssplit_psi_block<Store, SOLID, OFF32>(static_cast<const Store *>(B.pop[parity]), B.nbw, B.P, g,
+                                        p, b - first[l]);
 }
 
+// ONE: both passes in one launch; q.order holds each turn and its lattice.
 // At most 128 VGPRs: four waves per SIMD (the compiler's choice, 129, gave three).
-template <class Store, bool OFF32>
+template <class Store, bool SOLID, bool OFF32, bool ONE>
 __global__ void __launch_bounds__(kShiftThreads) __attribute__((amdgpu_waves_per_eu(4)))
     k_batch_split_collide(const BatchLattice *__restrict__ lats, const int *__restrict__ first,
-                          int nlat, int blk0, int blk1, int parity) {
-  const int b = blk0 + blockIdx.x;
-  if (b >= blk1) return;  // whole block: no barrier is left waiting
-  const int l = uniform(batch_block_lattice(first, nlat, b));
+                          int nlat, int blk0, int blk1, int parity, SplitPlan q) {
+  int b, l;
+  bool collide = true;
+  if constexpr (ONE) {
+    const int32_t turn = q.order[2 * (blockIdx.x >> 3)];
+    l = q.order[2 * (blockIdx.x >> 3) + 1];
+    if ((int)(blockIdx.x & 7) >= turn_count(turn)) return;
+    b = turn_first(turn) + (blockIdx.x & 7);
+    collide = turn_collide(turn);
+  } else {
+    b = blk0 + blockIdx.x;
+    if (b >= blk1) return;  // whole block: no barrier is left waiting
+    l = uniform(batch_block_lattice(first, nlat, b));
+  }
   ConstLattice &B = table_entry(lats, l);
   const Store *A = static_cast<const Store *>(B.pop[parity]);
-  Store *W = static_cast<Store *>(const_cast<void *>(B.pop[parity ^ 1]));
   const Geo g = B.g;
   const ShiftParams p = B.p;
-  if (p.has_solid)
-    ssplit_collide_block<Store, true, OFF32>(A, W, B.nbw, B.P, g, p, b - first[l], nullptr);
-  else
-    ssplit_collide_block<Store, false, OFF32>(A, W, B.nbw, B.P, g, p, b - first[l],
-                                              nullptr);
+  const int f0 = first[l];
+  if constexpr (ONE) {
+    if (p.sc) {
+      if (!shift_one_launch<Store, SOLID, OFF32>(A, B.nbw, B.P, g, p, q, f0, b - f0, collide))
+        return;
+    } else if (!collide) {  // no psi to write, but the flags stay in step
+      psi_publish(q, b);
+      return;
+    }
+  }
+  ssplit_collide_block<Store, SOLID, OFF32>(
+      A, static_cast<Store *>(const_cast<void *>(B.pop[parity ^ 1])), B.nbw, B.P, g, p, b - f0,
+      nullptr);
 }
 
 // The split pair as one persistent launch per step: the workgroups (all
@@ -459,16 +478,24 @@ inline hipError_t launch_batch_split_persistent(const BatchLattice *lats, const 
 
 // One step of the blocks [blk0, blk0 + nblk) of a batch on the split schedule;
 // psi: whether any of these members has Shan-Chen on (else pass 1 is skipped).
-template <class Store, bool OFF32>
+template <class Store, bool SOLID, bool OFF32>
 inline void launch_batch_split(const BatchLattice *lats, const int *first, int nlat, int blk0,
                                int nblk, int parity, bool psi, hipStream_t stream) {
   if (nblk <= 0) return;
-  const int grid = nblk;
+  const dim3 grid(nblk), block(kShiftThreads);
   if (psi)
-    hipLaunchKernelGGL((k_batch_split_psi<Store, OFF32>), dim3(grid), dim3(kShiftThreads), 0,
-                       stream, lats, first, nlat, blk0, blk0 + nblk, parity);
-  hipLaunchKernelGGL((k_batch_split_collide<Store, OFF32>), dim3(grid), dim3(kShiftThreads), 0,
-                     stream, lats, first, nlat, blk0, blk0 + nblk, parity);
+    hipLaunchKernelGGL((k_batch_split_psi<Store, SOLID, OFF32>), grid, block, 0, stream, lats,
+                       first, nlat, blk0, blk0 + nblk, parity);
+  hipLaunchKernelGGL((k_batch_split_collide<Store, SOLID, OFF32, false>), grid, block, 0, stream,
+                     lats, first, nlat, blk0, blk0 + nblk, parity, SplitPlan{});
+}
+
+// The same for all members in one launch of `norder` workgroups (q.order).
+template <class Store, bool SOLID, bool OFF32>
+inline void launch_batch_one(const BatchLattice *lats, const int *first, int nlat, int parity,
+                             const SplitPlan &q, int norder, hipStream_t stream) {
+  hipLaunchKernelGGL((k_batch_split_collide<Store, SOLID, OFF32, true>), dim3(norder),
+                     dim3(kShiftThreads), 0, stream, lats, first, nlat, 0, 0, parity, q);
 }
 
 }  // namespace dlbc

@@ -159,17 +159,21 @@ inline void split_order_lists(const Geo &g, int SB, int blk0, std::vector<int32_
 }
 
 // The turns of a launch over these lists: runs of consecutive blocks, psi in
-// front of every collide by `ahead` blocks.
+// front of every collide by `ahead` blocks.  With several lattices (`starts`:
+// their first blocks) no turn crosses from one to the next.
 inline std::vector<int32_t> split_order_merge(const std::vector<int32_t> &psi,
                                               const std::vector<int32_t> &col,
                                               const std::vector<int32_t> &need,
-                                              int ahead = kOrderAhead) {
+                                              int ahead = kOrderAhead,
+                                              const std::vector<int> &starts = {}) {
   std::vector<int32_t> out;
   out.reserve((psi.size() + col.size()) / 8 + (psi.size() + col.size()) / 64 + 32);
   size_t pp = 0, cp = 0;
-  auto run = [](const std::vector<int32_t> &v, size_t p) {
+  auto run = [&](const std::vector<int32_t> &v, size_t p) {
+    const auto next = std::upper_bound(starts.begin(), starts.end(), v[p]);
+    const int64_t end = next == starts.end() ? INT32_MAX : *next;
     int n = 1;
-    while (n < 8 && p + n < v.size() && v[p + n] == v[p] + n) ++n;
+    while (n < 8 && p + n < v.size() && v[p + n] == v[p] + n && v[p] + n < end) ++n;
     return n;
   };
   while (cp < col.size()) {

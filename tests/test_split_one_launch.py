@@ -16,6 +16,15 @@ def test_order_visits_every_block_and_never_waits_for_a_later_one(n, sites):
     assert D.lib().dlbc_selftest_split_order(*n, sites) == 0
 
 
+@pytest.fixture(scope="module")
+def D():
+    import dlbc_amd
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail("no GPU visible")
+    return dlbc_amd
+
+
 def _params(n, form, solid):
     rng = np.random.default_rng(sum(n))
     p = dict(d=3, q=19, gn=list(n), components=2, tau=[1.0, 0.9], eqDistForm=form,
@@ -38,8 +47,7 @@ def _same(a, b, what):
 @pytest.mark.parametrize("n", [(70, 90, 61), (2, 1250, 131), (16, 200, 128), (15, 211, 131),
                                (41, 3, 2620)], ids=str)
 @pytest.mark.parametrize("form,solid", [("BDist2", True), ("SecondOrder", False)])
-def test_f64_equals_oracle(n, form, solid):
-    import dlbc_amd as D
+def test_f64_equals_oracle(D, n, form, solid):
     from oracle.oracle import Oracle
     p = _params(n, form, solid)
     g, o = D.Lattice.from_params(p, schedule="split"), Oracle.from_params(p)
@@ -53,11 +61,10 @@ def test_f64_equals_oracle(n, form, solid):
                                        ("f32_shift", (13, 470, 256)), ("f16_shift", (24, 256, 256))],
                          ids=str)
 @pytest.mark.parametrize("solid", [True, False])
-def test_equals_two_launches(storage, n, solid):
+def test_equals_two_launches(D, storage, n, solid):
     """Any block order keeps two launches per step; both give the same bits,
     also in turn, over odd step counts, from a graph and where no collide wave
     waits for the psi it reads (each computes it)."""
-    import dlbc_amd as D
     p = _params(n, "BDist2", solid)
     a, b = (D.Lattice.from_params(p, storage=storage, schedule="split") for _ in range(2))
     b.set_block_order(8)
@@ -75,3 +82,31 @@ def test_equals_two_launches(storage, n, solid):
     a.step(1)
     b.step(1)
     _same(a, b, "no waiting")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage,solid", [("f32_shift", False), ("f32_shift", True),
+                                           ("f16_shift", False)])
+def test_batch_in_one_launch_equals_lattices_alone(D, storage, solid):
+    """A batch large enough for one launch per step: eager, graph and odd step
+    counts, and a member whose Shan-Chen force goes off and on in between."""
+    sizes = [(70, 83, 91), (4, 4, 4), (64, 96, 128), (33, 70, 31)]
+    ps = [_params(n, "BDist2", solid) for n in sizes]
+    alone, members = ([D.Lattice.from_params(p, storage=storage) for p in ps] for _ in range(2))
+    batch = D.Batch(members)
+    batch.set_config(8, 64, 512, 2)
+
+    def params(lat, p, on):
+        lat.set_params(p["tau"], p["gcc"], p.get("gwc"), None, None, p["eqDistForm"], "Exponential",
+                       on)
+
+    for k, graph, on in ((4, True, True), (3, False, True), (2, True, False), (1, False, False),
+                         (6, True, True), (1, True, True)):
+        for lats in (alone, members):
+            params(lats[2], ps[2], on)
+        batch.step(k, graph=graph)
+        for lat in alone:
+            lat.step(k)
+        batch.synchronize()
+    for a, b, n in zip(alone, members, sizes):
+        _same(a, b, n)
