@@ -19,6 +19,7 @@
 #include "kernels_march.hpp"
 #include "kernels_shifted.hpp"
 #include "kernels_split.hpp"
+#include "kernels_tile.hpp"
 #include "kernels_twopass.hpp"
 
 using namespace dlbc;
@@ -577,10 +578,26 @@ bool split_one_launch(const dlbc_gpu_ctx *c) {
   return c->geo.sites >= blocks * split_sites(c);
 }
 
+// Whether a step is one launch over small tiles (kernels_tile.hpp): D2Q9 with
+// Shan-Chen under the automatic schedule.  With one or two components in the
+// middle range, where both buffers stay in the memory-side cache and the
+// arithmetic of the border decides, two launches are faster (us per step, two
+// launches / one, two components: 400^2 18.9 / 17.1, 450^2 21.4 / 23.3, 850^2
+// 59 / 71, 1024^2 84 / 85, 1400^2 173 / 165, 2048^2 351 / 323); three and more
+// gain everywhere (300^2 21 / 19, 1024^2 154 / 149).  The kernel's 32-bit
+// offsets within a component need 9 sp 8 < 2^32.
+bool tile_step(const dlbc_gpu_ctx *c) {
+  if (c->schedule != DLBC_SCHED_AUTO || c->storage != DLBC_STORAGE_F64 || !c->p.sc || c->d != 2)
+    return false;
+  if (9 * 8 * c->geo.sp >= (int64_t)1 << 32) return false;
+  return c->C > 2 || c->geo.sites <= 160000 || c->geo.sites >= 1500000;
+}
+
 // The order and the flags of that launch, once per context.  Without the memory
 // for them the step stays at two launches.
 int split_ready(dlbc_gpu_ctx *c) {
-  if (c->order || effective_schedule(c) != DLBC_SCHED_SPLIT || !split_one_launch(c))
+  if (c->order || effective_schedule(c) != DLBC_SCHED_SPLIT || tile_step(c) ||
+      !split_one_launch(c))
     return DLBC_OK;
   std::vector<int32_t> o;
   try {
@@ -651,6 +668,23 @@ struct SplitStep {
   }
 };
 
+// One launch over tiles.
+template <class L, int C>
+struct TileStep {
+  static int run(dlbc_gpu_ctx *c, Timer *tm) {
+    if constexpr (std::is_same<L, D2Q9>::value) {
+      tm->before();
+      launch_tile_step<C>(static_cast<const double *>(c->popA), static_cast<double *>(c->popB),
+                          c->nbw, c->S, c->geo, c->p, c->stream);
+      tm->after();
+      std::swap(c->popA, c->popB);
+      return DLBC_OK;
+    } else {
+      return fail(c, DLBC_ERR_UNSUPPORTED, "tile step: D2Q9 only");
+    }
+  }
+};
+
 template <class L, int C>
 struct AdvectOnly {
   static int run(dlbc_gpu_ctx *c) {
@@ -709,6 +743,7 @@ int prepare(dlbc_gpu_ctx *c) {
 // the swap of the two population buffers, nothing else (so it can be captured).
 int step_once(dlbc_gpu_ctx *c, int sched, Timer *tm) {
   tm->slot = 0;
+  if (tile_step(c)) return dispatch<TileStep>(c, tm);
   if (sched == DLBC_SCHED_FUSED) return dispatch<FusedStep>(c, tm, (double *)nullptr);
   if (sched == DLBC_SCHED_SPLIT) return dispatch<SplitStep>(c, tm, (double *)nullptr);
   if (sched == DLBC_SCHED_MARCH) return dispatch<MarchStep>(c, tm, (double *)nullptr);
@@ -752,7 +787,7 @@ std::vector<unsigned char> graph_key(const dlbc_gpu_ctx *c, int sched) {
   };
   // the flag set and the buffer parity alternate together while the split
   // schedule takes one launch per step
-  const int ints[8] = {sched,         c->storage,    c->has_solid, c->target_blocks,
+  const int ints[9] = {c->schedule,   sched,         c->storage,    c->has_solid, c->target_blocks,
                        c->march_rows, c->march_hold, c->psi_set ^ (c->popA == c->bufX ? 0 : 1),
                        c->psi_polls};
   put(ints, sizeof ints);
@@ -1511,6 +1546,7 @@ int dlbc_gpu_step_timed(dlbc_gpu_ctx *c, int nsteps, double *elapsed_ms, double 
 const char *dlbc_gpu_kernel_name(const dlbc_gpu_ctx *c, int i) {
   if (!c) return "";
   const int sched = effective_schedule(c);
+  if (tile_step(c)) return i == 0 ? "tile_step" : "";
   if (sched == DLBC_SCHED_FUSED && c->storage != DLBC_STORAGE_F64)
     return i == 0 ? "tiled_d3q19_shifted" : "";
   if (sched == DLBC_SCHED_FUSED) return i == 0 ? "fused_d3q19" : "";
