@@ -19,6 +19,7 @@
 #include "kernels_init.hpp"
 #include "kernels_march.hpp"
 #include "kernels_shifted.hpp"
+#include "kernels_single.hpp"
 #include "kernels_split.hpp"
 #include "kernels_tile.hpp"
 #include "kernels_twopass.hpp"
@@ -493,8 +494,15 @@ struct TwoPassStep {
       tm->after();
     }
     tm->before();
-    hipLaunchKernelGGL((k_collide<L, C>), dim3(nb), dim3(256), 0, c->stream, A, B, c->mask, c->S,
-                       c->geo, c->p);
+    bool single = false;
+    if constexpr (C == 1 && L::q != 5) single = !c->p.sc && single_supported(c->geo, L::q);
+    if (single) {
+      if constexpr (C == 1 && L::q != 5)
+        launch_single<L>(A, B, c->nbw, c->geo, c->p, c->stream);
+    } else {
+      hipLaunchKernelGGL((k_collide<L, C>), dim3(nb), dim3(256), 0, c->stream, A, B, c->mask,
+                         c->S, c->geo, c->p);
+    }
     tm->after();
     (void)acc_ms;
     std::swap(c->popA, c->popB);

@@ -1,0 +1,102 @@
+// kernels_single.hpp -- one step of a single-component lattice without
+// Shan-Chen force (FP64, any connectivity): streaming, bounce-back, body force
+// and BGK collision in one launch.
+//
+// The step reads and writes each population once.  One lane per site: its
+// neighbours' places come from six offsets set up once (nbr_offsets), the solid
+// neighbourhood from one word, and every access takes a scalar base and a 32-bit
+// lane offset.  (The general kernel, k_collide, wraps and multiplies every
+// neighbour's coordinates and reads its mask byte.)  us per step, k_collide /
+// here: D2Q9 64^2 4.6 / 3.4, 700^2 with plates 16.6 / 14.5; D3Q19 32^3 6.8 / 5.3,
+// 70x45x98 with plates 23.3 / 18.8, 256^3 940 / 873 (5.8 TB/s, a plain copy 5.7),
+// 256^3 with solid spheres 1307 / 858 (solid lanes write their lines whole).
+//
+// Per-site arithmetic is the shared code of the other schedules.
+#pragma once
+
+#include "kernels_split.hpp"
+
+namespace dlbc {
+
+// Threads of a workgroup: one wave, so that small lattices reach every CU.
+constexpr int kSingleThreads = 64;
+
+// Nontemporal stores where the two buffers exceed the memory-side cache: 256^3 906
+// without and 873 us with, 160^3 with plates 219 and 211; 70x45x98, which stays
+// in it, 18.8 and 21.0.
+constexpr int64_t kSingleCached = 256ll << 20;
+
+// Whether the kernel serves a lattice: neighbours one site away on every axis
+// (not D1Q5), and 32-bit byte offsets.
+inline bool single_supported(const Geo &g, int q) {
+  return q != 5 && (int64_t)q * 8 * g.sp < (int64_t)1 << 32;
+}
+
+template <class L, bool SOLID, bool NT>
+__global__ void __launch_bounds__(kSingleThreads)
+    k_single(const double *__restrict__ A, double *__restrict__ B,
+             const uint32_t *__restrict__ nbw, Geo g, StepParams p) {
+  constexpr int Q = L::q, D = L::d;
+  const int s = blockIdx.x * kSingleThreads + threadIdx.x;
+  if (s >= g.sites) return;
+  // a solid site's lane stores the site's own populations again, so that whole
+  // cache lines are written; a line of solid sites only is left alone (as in
+  // k_split_collide)
+  uint32_t sw = SOLID ? nbw[s] : 0u;
+  const bool solid_site = sw >> 31;
+  if (SOLID && line_all_solid<16>(solid_site)) return;
+  if (solid_site) sw = (1u << Q) - 1u;
+  int x, y, z;
+  lane_coords(s, g, x, y, z);
+  const NbrOffsets o = nbr_offsets(g, x, y, z);
+  auto place = [](int site) {  // tile_elem<Q> in 32 bits
+    return (uint32_t)site + __umul24((uint32_t)site >> 6, 64u * (Q - 1));
+  };
+  double n[Q];
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    const int src = nbr_site(s, o, -L::c[i][0], -L::c[i][1], -L::c[i][2]);
+    const int b = L::bounce[i], lo = SOLID && b < i ? b : i;
+    const bool bb = SOLID && ((sw >> b) & 1u);
+    n[i] = at<true>(A + 64 * lo, 64 * ((bb ? b : i) - lo) + place(bb ? s : src));
+  }
+  const double rho = density<L>(n);
+  double F[D], wv[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) F[d] = 0.0;
+  const double total = total_density<1>([&](int) { return rho; });
+  if (p.eq_form == kBDist2) {
+    double mom[D];
+    first_moment<L>(n, mom);
+    weighted_velocity<L, 1>([&](int, int d) { return mom[d]; }, total, p, wv);
+  }
+  auto out = [&](int i, double v) {
+    double *to = elem<true>(B + 64 * i, place(s));
+    const double w = SOLID && solid_site ? n[L::bounce[i]] : v;
+    if (NT)
+      __builtin_nontemporal_store(w, to);
+    else
+      *to = w;
+  };
+  if constexpr (Q == 19)
+    collide_d3q19_streamed(0, n, rho, total, F, wv, p, out);
+  else
+    collide_component<L>(0, n, rho, total, F, wv, p, out);
+}
+
+template <class L>
+inline void launch_single(const double *A, double *B, const uint32_t *nbw, const Geo &g,
+                          const StepParams &p, hipStream_t stream) {
+  const dim3 grid((g.sites + kSingleThreads - 1) / kSingleThreads), block(kSingleThreads);
+  const bool nt = 2 * 8 * L::q * g.sp > kSingleCached;
+  if (p.has_solid && nt)
+    hipLaunchKernelGGL((k_single<L, true, true>), grid, block, 0, stream, A, B, nbw, g, p);
+  else if (p.has_solid)
+    hipLaunchKernelGGL((k_single<L, true, false>), grid, block, 0, stream, A, B, nbw, g, p);
+  else if (nt)
+    hipLaunchKernelGGL((k_single<L, false, true>), grid, block, 0, stream, A, B, nbw, g, p);
+  else
+    hipLaunchKernelGGL((k_single<L, false, false>), grid, block, 0, stream, A, B, nbw, g, p);
+}
+
+}  // namespace dlbc
