@@ -759,15 +759,50 @@ int step_once(dlbc_gpu_ctx *c, int sched, Timer *tm) {
   return dispatch<TwoPassStep>(c, tm, (double *)nullptr);
 }
 
+// Steps that one launch takes: several on small single-component D2Q9 lattices
+// without Shan-Chen force (kernels_single.hpp), else 1.  A workgroup per CU takes
+// eight; beyond, 16 x 16 tiles and four steps, while more than one round of them
+// still beats single steps.  us per step, single (eager / graph), four, eight:
+// 64^2 4.3 / 2.9, 2.4, 1.85; 128^2 4.5 / 3.4, 2.6, 2.0; 192^2 4.9 / 4.1, 3.1, 5.0;
+// 256^2 5.7 / 5.0, 3.4, 6.6; 300^2 6.5 / 6.1, 5.2; 400^2 8.7 / 8.5, 7.0; 512^2 8.3,
+// 9.3.
+int steps_per_launch(const dlbc_gpu_ctx *c) {
+  if (c->schedule != DLBC_SCHED_AUTO || c->storage != DLBC_STORAGE_F64 || c->d != 2 ||
+      c->C != 1 || c->p.sc)
+    return 1;
+  auto tiles = [&](int t) { return (int64_t)((c->n[0] + t - 1) / t) * ((c->n[1] + t - 1) / t); };
+  if (tiles(8) <= 256) return multi_steps<8>();
+  if (tiles(16) <= 256 || (tiles(16) <= 650 && c->geo.sites >= 80000)) return multi_steps<16>();
+  return 1;
+}
+
+// nsteps steps: launches on the library stream and swaps of the two population
+// buffers, nothing else (so they can be captured).
+int advance(dlbc_gpu_ctx *c, int sched, int nsteps, Timer *tm) {
+  const int per = steps_per_launch(c);
+  int t = 0;
+  for (; per > 1 && t + per <= nsteps; t += per) {
+    const double *A = static_cast<const double *>(c->popA);
+    double *B = static_cast<double *>(c->popB);
+    if (per == multi_steps<8>())
+      launch_single_multi<8>(A, B, c->nbw, c->geo, c->p, c->stream);
+    else
+      launch_single_multi<16>(A, B, c->nbw, c->geo, c->p, c->stream);
+    std::swap(c->popA, c->popB);
+  }
+  for (; t < nsteps; ++t) {
+    const int rc = step_once(c, sched, tm);
+    if (rc) return rc;
+  }
+  return DLBC_OK;
+}
+
 int do_steps(dlbc_gpu_ctx *c, int nsteps, Timer *tm) {
   int rc = prepare(c);
   if (!rc) rc = split_ready(c);
   if (rc) return rc;
-  const int sched = effective_schedule(c);
-  for (int t = 0; t < nsteps; ++t) {
-    rc = step_once(c, sched, tm);
-    if (rc) return rc;
-  }
+  rc = advance(c, effective_schedule(c), nsteps, tm);
+  if (rc) return rc;
   HIPCHK(c, hipGetLastError());
   return DLBC_OK;
 }
@@ -1534,7 +1569,8 @@ int dlbc_gpu_step(dlbc_gpu_ctx *c, int nsteps) {
   return do_steps(c, nsteps, &tm);
 }
 
-// Steps per captured graph (even).
+// Steps per captured graph (even, and an even number of launches where a launch
+// takes four or eight).
 constexpr int kGraphSteps = 32;
 
 int dlbc_gpu_step_graph(dlbc_gpu_ctx *c, int nsteps) {
@@ -1563,8 +1599,7 @@ int dlbc_gpu_step_graph(dlbc_gpu_ctx *c, int nsteps) {
       void *const a = c->popA, *const b = c->popB;
       hipGraph_t g = nullptr;
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      int rcc = 0;
-      for (int k = 0; k < kGraphSteps && !rcc; ++k) rcc = step_once(c, sched, &tm);
+      const int rcc = advance(c, sched, kGraphSteps, &tm);
       const hipError_t ec = hipStreamEndCapture(c->stream, &g);
       c->popA = a;  // captured, not run
       c->popB = b;
@@ -1581,10 +1616,8 @@ int dlbc_gpu_step_graph(dlbc_gpu_ctx *c, int nsteps) {
     for (; t + kGraphSteps <= nsteps; t += kGraphSteps)
       HIPCHK(c, hipGraphLaunch(c->graph[par], c->stream));
   }
-  for (; t < nsteps; ++t) {
-    rc = step_once(c, sched, &tm);
-    if (rc) return rc;
-  }
+  rc = advance(c, sched, nsteps - t, &tm);
+  if (rc) return rc;
   HIPCHK(c, hipGetLastError());
   return DLBC_OK;
 }

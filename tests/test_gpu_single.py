@@ -37,3 +37,29 @@ def test_single_component_equals_oracle(D, dq, n, form, solid):
     o.run(4)
     x, y = a.population(0), o.population(0)
     assert np.array_equal(x.view(np.uint64), y.view(np.uint64))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [(2, 2), (5, 3), (8, 8), (23, 9), (24, 25), (64, 64), (128, 128),
+                               (129, 121), (256, 250), (300, 300), (2000, 3)], ids=str)
+@pytest.mark.parametrize("form", ["SecondOrder", "BDist2"])
+@pytest.mark.parametrize("solid", [False, True])
+def test_several_steps_in_one_launch_equal_oracle(D, n, form, solid):
+    """Step counts below, at and past a launch's eight or four steps, eager and
+    from a graph, on lattices smaller than a workgroup's 24 x 24 sites, of whole
+    tiles, and with tiles over the end of an axis."""
+    from oracle.oracle import Oracle
+    rng = np.random.default_rng(n[0])
+    p = dict(d=2, q=9, gn=list(n), components=1, tau=[0.9], eqDistForm=form,
+             globalAcc=[0.0, 1e-5], fluidInit=["EqDistPerturb"], fluidDensities=[[1.0]],
+             fluidPerturb=[0.02], randomReseed=[True], randomSeed=[12])
+    if solid:
+        p["maskArray"] = (rng.random(n) < 0.1).astype(np.int32)
+    a, o = D.Lattice.from_params(p), Oracle.from_params(p)
+    done = 0
+    for k, graph in ((3, False), (8, False), (13, False), (39, True)):
+        a.step(k, graph=graph)
+        done += k
+    o.run(done)
+    x, y = a.population(0), o.population(0)
+    assert np.array_equal(x.view(np.uint64), y.view(np.uint64))
