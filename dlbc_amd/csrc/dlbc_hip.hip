@@ -572,6 +572,11 @@ int split_sites(const dlbc_gpu_ctx *c) {
   return c->storage == DLBC_STORAGE_F64 ? kSplitThreads / 2 : kShiftSites;
 }
 
+// Blocks of a strip's plane in the one-launch order.
+int order_strip(int storage) {
+  return storage == DLBC_STORAGE_F16_SHIFT ? kOrderStripF16 : kOrderStrip;
+}
+
 // Whether a Shan-Chen step of the split schedule is one launch.  us per step,
 // two launches against one: FP64 48^3 22 / 34, 64^3 42.6 / 42.5, 72^3 63.5 /
 // 61.3, 96^3 148 / 135, 256^3 2960 / 2385; FP32 80^3 42 / 48, 96^3 70 / 73,
@@ -610,7 +615,7 @@ int split_ready(dlbc_gpu_ctx *c) {
     return DLBC_OK;
   std::vector<int32_t> o;
   try {
-    o = split_order(c->geo, split_sites(c));
+    o = split_order(c->geo, split_sites(c), order_strip(c->storage));
   } catch (const std::bad_alloc &) {
     c->one_launch_off = true;
     return DLBC_OK;
@@ -1876,7 +1881,8 @@ int64_t dlbc_selftest_split_order(int nx, int ny, int nz, int block_sites) {
   g.sites = (int)sites;
   g.sp = (sites + 63) / 64 * 64;
   geo_set_divisors(g);
-  return split_order_faults(g, block_sites, split_order(g, block_sites));
+  return split_order_faults(g, block_sites, split_order(g, block_sites)) +
+         split_order_faults(g, block_sites, split_order(g, block_sites, kOrderStripF16));
 }
 
 int dlbc_selftest_set_psi_polls(dlbc_gpu_ctx *c, int polls) {
@@ -2067,7 +2073,8 @@ int batch_split_ready(dlbc_batch *b) {
   try {
     std::vector<int32_t> psi, col, need;
     for (size_t l = 0; l < b->ctx.size(); ++l)
-      split_order_lists(b->ctx[l]->geo, kShiftSites, b->h_first[l], psi, col, need);
+      split_order_lists(b->ctx[l]->geo, kShiftSites, b->h_first[l], psi, col, need,
+                        order_strip(b->storage));
     for (int32_t t : split_order_merge(psi, col, need, kOrderAhead, b->h_first)) {
       const auto next = std::upper_bound(b->h_first.begin(), b->h_first.end(), turn_first(t));
       turns.push_back(t);
