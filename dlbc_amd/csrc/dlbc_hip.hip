@@ -562,7 +562,7 @@ int effective_schedule(const dlbc_gpu_ctx *c) {
   // FP16 0.84 against 2.0); the tiled kernel (FUSED) remains selectable
   if (c->storage != DLBC_STORAGE_F64) return DLBC_SCHED_SPLIT;
   // D3Q19 two-component FP64: the lane-per-component two-pass kernels are the
-  // fastest measured schedule (256^3 channel: 2.57 ms/step vs 4.20 ms fused)
+  // fastest measured schedule (256^3 channel: 2.37 ms/step vs 4.20 ms fused)
   if (c->d == 3 && c->C == 2) return DLBC_SCHED_SPLIT;
   return DLBC_SCHED_TWO_PASS;
 }
@@ -579,9 +579,9 @@ int order_strip(int storage) {
 
 // Whether a Shan-Chen step of the split schedule is one launch.  us per step,
 // two launches against one: FP64 48^3 22 / 34, 64^3 42.6 / 42.5, 72^3 63.5 /
-// 61.3, 96^3 148 / 135, 256^3 2960 / 2385; FP32 80^3 42 / 48, 96^3 70 / 73,
-// 190x151x117 with solids 292 / 276, 256^3 1390 / 1157; FP16 without solids
-// 128^3 91 / 90, 256^3 719 / 680, 384^3 2570 / 2330.  FP16 with solids, whose
+// 61.3, 96^3 148 / 135, 256^3 2960 / 2254; FP32 80^3 42 / 48, 96^3 70 / 73,
+// 190x151x117 with solids 292 / 249, 256^3 1390 / 1120; FP16 without solids
+// 128^3 91 / 90, 256^3 719 / 657, 384^3 2570 / 2310.  FP16 with solids, whose
 // collide is bound by its instructions and whose psi then runs at the collide's
 // four waves per SIMD, 836 / 943 at 256^3: two launches.
 bool split_one_launch(const dlbc_gpu_ctx *c) {

@@ -384,7 +384,7 @@ __global__ void __launch_bounds__(kShiftThreads) __attribute__((amdgpu_waves_per
     const int32_t turn = q.order[2 * (blockIdx.x >> 3)];
     l = q.order[2 * (blockIdx.x >> 3) + 1];
     if ((int)(blockIdx.x & 7) >= turn_count(turn)) return;
-    b = turn_first(turn) + (blockIdx.x & 7);
+    b = turn_first(turn) + (int)(blockIdx.x & 7) * turn_stride(turn);
     collide = turn_collide(turn);
   } else {
     b = blk0 + blockIdx.x;

@@ -526,7 +526,7 @@ __global__ void __launch_bounds__(kSplitThreads)
   if constexpr (ONE) {
     const int32_t turn = q.order[blockIdx.x >> 3];
     if ((int)(blockIdx.x & 7) >= turn_count(turn)) return;
-    blk = turn_first(turn) + (blockIdx.x & 7);
+    blk = turn_first(turn) + (int)(blockIdx.x & 7) * turn_stride(turn);
     const bool is_psi = !turn_collide(turn);
     if (is_psi || !psi_wait(q, g, SB, 0, blk)) {
       // the wave's part of the block's psi, or (not waited for any longer) all
@@ -787,7 +787,7 @@ __global__ void __launch_bounds__(kShiftThreads) __attribute__((amdgpu_waves_per
   if constexpr (ONE) {
     const int32_t turn = q.order[blockIdx.x >> 3];
     if ((int)(blockIdx.x & 7) >= turn_count(turn)) return;
-    blk = turn_first(turn) + (blockIdx.x & 7);
+    blk = turn_first(turn) + (int)(blockIdx.x & 7) * turn_stride(turn);
     if (!shift_one_launch<Store, SOLID, OFF32>(A, nbw, P, g, p, q, 0, blk, turn_collide(turn)))
       return;
   } else {

@@ -27,25 +27,32 @@
 namespace dlbc {
 
 // Blocks of a strip's plane, blocks that psi is ahead, and turns of psi in a
-// row.  FP64, 256^3 without solids: 2440 us per step with strips of 128 blocks
-// and psi and collide turns one by one, 2385 with psi in rows of eight turns
-// (one by one, workgroups that did nothing at all in the psi turns' place
-// slowed the collide workgroups by a quarter).  Strips of 64, 256 and a whole
-// plane (512 blocks): 2510, 2500 and 2610.  Psi 512 blocks ahead: 2830 (collide
-// workgroups wait: some 1280 workgroups are resident), 768 to 1024: the same,
-// 1500: 2510.
+// row.  FP64, 256^3 without solids, us per step.  Psi and collide turns one by
+// one 2440, psi in rows of eight turns 2385 (one by one, workgroups that did
+// nothing at all in the psi turns' place slowed the collide workgroups by a
+// quarter).  With the spans below: strips of 128, 192 and 256 blocks 2254, 2285
+// and 2254 (a whole plane, before them: 2610 against 2385); psi 896, 1024 and
+// 1280 blocks ahead 2250, 2254 and 2265, at 128^3 in FP32 163, 151 and 148 (some
+// 1280 workgroups are resident: closer, and collide workgroups wait).
 // A FP16 block has half the bytes, and strips of twice the blocks lose less at
 // their edges: 384^3 without solids 2405 us with 128, 2335 with 256, 2700 with 512.
 constexpr int kOrderStrip = 128, kOrderStripF16 = 256, kOrderAhead = 1024, kOrderRow = 8;
 
 // A turn: what eight consecutive workgroups do (workgroup b runs on XCD b % 8, so
 // every XCD gets both kinds in equal parts).  Workgroup j < turn_count takes
-// block turn_first + j, the others nothing.
-constexpr int32_t order_turn(int first, int count, bool collide) {
-  return first << 5 | count << 1 | (collide ? 1 : 0);
+// block turn_first + j * turn_stride, the others nothing.  Where 8 kOrderSpan
+// consecutive blocks stand in a row, kOrderSpan turns give each XCD kOrderSpan
+// of them, so that the psi rows that neighbouring blocks share are in its L2:
+// FP64 256^3 2435 us with turns of consecutive blocks, 2285 with spans of 4,
+// 2274 with 8, 2286 with 16; 190x151x117 with solids FP64 569, 536, 535 and 530,
+// FP32 278, 264, 251 and 261.
+constexpr int kOrderSpan = 8;
+constexpr int32_t order_turn(int first, int count, bool spread, bool collide) {
+  return first << 6 | count << 2 | (spread ? 2 : 0) | (collide ? 1 : 0);
 }
-__host__ __device__ inline int turn_first(int32_t t) { return t >> 5; }
-__host__ __device__ inline int turn_count(int32_t t) { return t >> 1 & 15; }
+__host__ __device__ inline int turn_first(int32_t t) { return t >> 6; }
+__host__ __device__ inline int turn_count(int32_t t) { return t >> 2 & 15; }
+__host__ __device__ inline int turn_stride(int32_t t) { return (t & 2) ? kOrderSpan : 1; }
 __host__ __device__ inline bool turn_collide(int32_t t) { return t & 1; }
 
 // The blocks whose psi a collide of block blk reads, as intervals [lo, hi] of
@@ -170,32 +177,40 @@ inline std::vector<int32_t> split_order_merge(const std::vector<int32_t> &psi,
                                               const std::vector<int> &starts = {}) {
   std::vector<int32_t> out;
   out.reserve((psi.size() + col.size()) / 8 + (psi.size() + col.size()) / 64 + 32);
-  size_t pp = 0, cp = 0;
-  auto run = [&](const std::vector<int32_t> &v, size_t p) {
+  // consecutive blocks from place p on, at most `most`
+  auto run = [&](const std::vector<int32_t> &v, size_t p, int most) {
     const auto next = std::upper_bound(starts.begin(), starts.end(), v[p]);
     const int64_t end = next == starts.end() ? INT32_MAX : *next;
     int n = 1;
-    while (n < 8 && p + n < v.size() && v[p + n] == v[p] + n && v[p] + n < end) ++n;
+    while (n < most && p + n < v.size() && v[p + n] == v[p] + n && v[p] + n < end) ++n;
     return n;
   };
-  while (cp < col.size()) {
-    const int c = run(col, cp);
-    int n = 0;
-    for (int k = 0; k < c; ++k) n = std::max(n, need[cp + k]);
-    const bool due = pp < (size_t)n + ahead;
-    while (due && pp < psi.size() && pp < (size_t)n + ahead + 8 * (kOrderRow - 1)) {
-      const int k = run(psi, pp);
-      out.push_back(order_turn(psi[pp], k, false));
-      pp += k;
+  // the turns of the next run of v, which is returned; need of a turn before it
+  size_t pp = 0;
+  auto put = [&](const std::vector<int32_t> &v, size_t p, bool collide, auto before) {
+    constexpr int whole = 8 * kOrderSpan;
+    if (kOrderSpan > 1 && run(v, p, whole) == whole) {
+      for (int k = 0; k < kOrderSpan; ++k) {
+        before(p, whole);
+        out.push_back(order_turn(v[p] + k, 8, true, collide));
+      }
+      return whole;
     }
-    out.push_back(order_turn(col[cp], c, true));
-    cp += c;
-  }
-  while (pp < psi.size()) {
-    const int k = run(psi, pp);
-    out.push_back(order_turn(psi[pp], k, false));
-    pp += k;
-  }
+    const int n = run(v, p, 8);
+    before(p, n);
+    out.push_back(order_turn(v[p], n, false, collide));
+    return n;
+  };
+  auto nothing = [](size_t, int) {};
+  for (size_t cp = 0; cp < col.size();)
+    cp += put(col, cp, true, [&](size_t p, int c) {
+      int n = 0;
+      for (int k = 0; k < c; ++k) n = std::max(n, need[p + k]);
+      const bool due = pp < (size_t)n + ahead;
+      while (due && pp < psi.size() && pp < (size_t)n + ahead + 8 * (kOrderRow - 1))
+        pp += put(psi, pp, false, nothing);
+    });
+  while (pp < psi.size()) pp += put(psi, pp, false, nothing);
   return out;
 }
 
@@ -218,7 +233,7 @@ inline int64_t split_order_faults(const Geo &g, int SB, const std::vector<int32_
   int64_t bad = 0;
   for (size_t p = 0; p < o.size(); ++p)
     for (int j = 0; j < turn_count(o[p]); ++j) {
-      const int b = turn_first(o[p]) + j, k = turn_collide(o[p]) ? 1 : 0;
+      const int b = turn_first(o[p]) + j * turn_stride(o[p]), k = turn_collide(o[p]) ? 1 : 0;
       if (b < 0 || b >= nb || turn_count(o[p]) > 8 || at[k][b] != -1) {
         ++bad;
         continue;
