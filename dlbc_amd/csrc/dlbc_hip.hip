@@ -119,8 +119,9 @@ int ensure_scratch(dlbc_gpu_ctx *c, size_t bytes) {
 inline int blocks_for(int64_t n, int bs) { return (int)((n + bs - 1) / bs); }
 
 // Block order of the split kernels (split_block): chunk -1 picks it from the
-// geometry, 0 keeps site order, K > 0 gives the XCDs K blocks per turn.  The
-// automatic choice is site order (see kSplitAutoChunk).
+// geometry, 0 keeps the library's order (site order, or the table of the
+// one-launch step), K > 0 gives the XCDs K blocks per turn in two launches.
+// The automatic choice is 0 (see kSplitAutoChunk).
 void apply_block_order(dlbc_gpu_ctx *c, int chunk) {
   const int spb = c->storage == DLBC_STORAGE_F64 ? kSplitThreads / 2 : kShiftSites;
   if (chunk < 0) {

@@ -418,7 +418,8 @@ __global__ void __launch_bounds__(kShiftThreads) __attribute__((amdgpu_waves_per
 // as the two launches.  psi is uniform, and nothing returns from the kernel
 // before the barrier, so every workgroup reaches it.  (Contiguous runs of
 // blocks per workgroup instead were slower: 8.35 against 8.07 ms per step on
-// the 256-lattice ensemble.)
+// the 256-lattice ensemble, before the populations lay in tiles; 7.75 ms now,
+// and 5.41 for the one-launch form above.)
 template <class Store, bool OFF32>
 __global__ void __launch_bounds__(kShiftThreads) __attribute__((amdgpu_waves_per_eu(4)))
     k_batch_split_persistent(const BatchLattice *__restrict__ lats, const int *__restrict__ first,

@@ -21,8 +21,8 @@
 // When a block's sites lie in one z-row (n_z a multiple of the block's
 // sites), pass 2 stages the nine psi rows around the block in LDS with
 // coalesced loads issued after the pulls, instead of gathering 19 scattered
-// psi values per lane: 2.32 against 2.46 ms per FP64 collide at 256^3, with
-// the same bits.
+// psi values per lane: 2.32 against 2.46 ms per FP64 collide at 256^3 (two
+// launches, one array per population), with the same bits.
 //
 // Per-site arithmetic is the shared code of the other schedules (density,
 // sc_force, total_density, weighted_velocity, collide_component), so all
@@ -45,7 +45,8 @@ constexpr int kShiftSites = 256;
 
 // Grid of a split launch over `sites`: threads / 2 sites per block.  (A grid
 // that gave each XCD one contiguous run of sites, an eighth of the lattice,
-// measured slower: 3.76 against 3.43 ms per FP64 step at 256^3.)
+// measured slower: 3.76 against 3.43 ms per FP64 step of two launches at
+// 256^3, with one array per population.)
 inline int split_grid(int64_t sites, int threads = kSplitThreads) {
   return (int)((sites + threads / 2 - 1) / (threads / 2));
 }
@@ -63,9 +64,9 @@ __device__ inline int split_block(const Geo &g, int b) {
   return ((j / K) * 8 + (b & 7)) * K + j % K;
 }
 
-// Whether the library picks an XCD block order by itself (an eighth of an
-// x-plane per turn) or keeps site order.  Site order: on the 256^3 channel
-// (FP64) chunks of 8 to 256 blocks cut the collide pass's L2 misses by a
+// Whether the library picks an XCD block order for the two launches by itself
+// (an eighth of an x-plane per turn) or keeps site order.  Site order: on the
+// 256^3 channel (FP64, one array per population) chunks of 8 to 256 blocks cut the collide pass's L2 misses by a
 // quarter (FETCH_SIZE 3.49 -> 2.60 GiB at K = 64) yet ran 2.53-2.74 ms
 // against 2.46 ms in site order.
 constexpr bool kSplitAutoChunk = false;

@@ -298,7 +298,7 @@ class Lattice:
 
     def step(self, nsteps=1, graph=False):
         """nsteps time steps (src/main.d:174-200); graph=True replays them
-        from a captured two-step HIP graph (same bits, less launch latency)."""
+        from a captured HIP graph (same bits, less launch latency)."""
         fn = lib().dlbc_gpu_step_graph if graph else lib().dlbc_gpu_step
         self._check(fn(self.h, int(nsteps)), "step")
 
@@ -333,7 +333,7 @@ class Lattice:
         self._check(lib().dlbc_gpu_set_march(self.h, int(rows), int(hold)), "set_march")
 
     def set_block_order(self, chunk):
-        """Split schedule: K > 0 blocks per XCD turn, 0 site order, -1 automatic."""
+        """Split schedule: K > 0 blocks per XCD turn, 0 the library's order, -1 automatic."""
         self._check(lib().dlbc_gpu_set_block_order(self.h, int(chunk)), "set_block_order")
 
     @property
@@ -457,7 +457,7 @@ class Lattice:
 
 class Batch:
     """Independent D3Q19 two-component lattices (shifted storage, any size)
-    advanced together: one persistent launch per step (dlbc_batch_*)."""
+    advanced together, in one or two launches per step (dlbc_batch_*)."""
 
     def __init__(self, lattices):
         self.members = list(lattices)  # keep the contexts alive
@@ -486,7 +486,7 @@ class Batch:
 
     def set_config(self, tile_y, chunk, workgroups, kernel=0):
         """kernel: 0 / 1 the tiled persistent kernel (with / without solids),
-        2 the split pair, 3 the split pair as one persistent launch."""
+        2 the split kernels, 3 the split pair as one persistent launch."""
         self._check(lib().dlbc_batch_set_config(self.h, tile_y, chunk, workgroups, kernel),
                     "set_config")
 

@@ -125,7 +125,9 @@ int dlbc_gpu_step(dlbc_gpu_ctx *ctx, int nsteps);
 /* As dlbc_gpu_step, with the steps replayed from a captured HIP graph of 32
  * steps (one graph per buffer parity; the remainder of nsteps runs eagerly).
  * Same results bit for bit; for small lattices, whose steps are bound by
- * launch latency (D2Q9 64x64: 3.9 instead of 4.7 us per step).  The graphs are
+ * launch latency (two-fluid D3Q19 32^3: 9.8 instead of 10.6 us per step;
+ * single-component D2Q9, which takes up to eight steps per launch, is as fast
+ * eagerly).  The graphs are
  * captured on first use and again when the schedule, launch shape, block
  * order, parameters or solid state changed since.
  * Replaces the same runTimeloop body as dlbc_gpu_step (src/main.d:174-200). */
@@ -156,8 +158,9 @@ int dlbc_gpu_get_schedule(const dlbc_gpu_ctx *ctx);
 int dlbc_gpu_set_launch(dlbc_gpu_ctx *ctx, int min_workgroups);
 /* Block order of the split schedule: chunk K > 0 gives the GPU's XCDs K
  * consecutive blocks of sites each in turn (block b runs on XCD b mod 8), so
- * neighbouring rows share an XCD's L2; 0 keeps site order; -1 lets the
- * library choose.  The results do not depend on it.  No counterpart in the
+ * neighbouring rows share an XCD's L2, in two launches per step; 0 keeps the
+ * library's order (site order, or on large lattices the order of the one-launch
+ * step); -1 lets the library choose (0).  The results do not depend on it.  No counterpart in the
  * reference. */
 int dlbc_gpu_set_block_order(dlbc_gpu_ctx *ctx, int chunk);
 /* Launch shape of the march schedule: rows = z-rows per workgroup (1, or 2
@@ -254,8 +257,8 @@ int64_t dlbc_gpu_device_bytes(const dlbc_gpu_ctx *ctx);
  * --------------------------------------------------------------------- */
 
 /* ------------------------------------------------------------------------
- * Batches: many independent lattices advanced by one persistent launch per
- * step.  No counterpart in the reference (one lattice per run); each member
+ * Batches: many independent lattices advanced together, by one launch (or
+ * two) per step.  No counterpart in the reference (one lattice per run); each member
  * is an ordinary context (its own parameters, uploads, fields, reductions)
  * created with DLBC_STORAGE_F32_SHIFT or F16_SHIFT, D3Q19, two components, of
  * any size n >= 4.  The caller keeps the members alive while the batch
@@ -267,9 +270,10 @@ int dlbc_batch_create(dlbc_batch **out, dlbc_gpu_ctx *const *lattices, int n);
 /* Tile height (4 or 8 rows of 32 sites), x-chunk length (planes), number of
  * workgroups of the persistent launch and kernel: 0 the tiled kernel
  * (solid-capable, 128 VGPRs), 1 the tiled kernel for batches without solid
- * sites (more loads in flight), 2 the split pair (a psi launch and a
- * stream/force/collide launch per step over all members; tile, chunk and
- * workgroups do not apply), 3 the split pair as one persistent cooperative
+ * sites (more loads in flight), 2 the split kernels (psi and
+ * stream/force/collide over all members, in one launch per step when the
+ * batch is large and in two when it is small; tile, chunk and workgroups do
+ * not apply), 3 the split pair as one persistent cooperative
  * launch per step (a grid barrier between the passes; every workgroup
  * resident; not captured into graphs).  Defaults 8, whole lattice, 512, 0. */
 int dlbc_batch_set_config(dlbc_batch *b, int tile_y, int chunk, int workgroups, int kernel);
@@ -278,7 +282,7 @@ int dlbc_batch_get_config(const dlbc_batch *b, int *out /*4*/);
  * current state (reads it, writes only the buffer the next step overwrites)
  * and keep the fastest; out receives it, best_ms its launch time. */
 int dlbc_batch_autotune(dlbc_batch *b, int *out /*4*/, double *best_ms);
-/* nsteps steps, one launch per step (two for kernel 2); with use_graph
+/* nsteps steps, one launch per step (kernel 2: one or two); with use_graph
  * pairs of steps are replayed from a captured HIP graph (not for kernel 3). */
 int dlbc_batch_step(dlbc_batch *b, int nsteps, int use_graph);
 /* The same steps as one launch per member and step (the per-lattice loop). */
