@@ -75,8 +75,8 @@ struct dlbc_gpu_ctx {
   // scratch for reductions and transfers
   double *scratch = nullptr;
   size_t scratch_bytes = 0;
-  // dlbc_gpu_step_graph: two captured steps per buffer parity, and the host
-  // state their kernel arguments were captured from
+  // dlbc_gpu_step_graph: kGraphSteps captured steps per buffer parity, and the
+  // host state their kernel arguments were captured from
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   std::vector<unsigned char> graph_key;
 };
@@ -835,11 +835,12 @@ std::vector<unsigned char> graph_key(const dlbc_gpu_ctx *c, int sched) {
     const auto *b = static_cast<const unsigned char *>(p);
     k.insert(k.end(), b, b + n);
   };
-  // the flag set and the buffer parity alternate together while the split
-  // schedule takes one launch per step
-  const int ints[9] = {c->schedule,   sched,         c->storage,    c->has_solid, c->target_blocks,
-                       c->march_rows, c->march_hold, c->psi_set ^ (c->popA == c->bufX ? 0 : 1),
-                       c->psi_polls};
+  // while a step is one launch of the split schedule, the flag set and the buffer
+  // parity alternate together; no other step reads the flags
+  const bool one = sched == DLBC_SCHED_SPLIT && split_one_launch(c);
+  const int flags = one ? 1 + (c->psi_set ^ (c->popA == c->bufX ? 0 : 1)) : 0;
+  const int ints[9] = {c->schedule,   sched,         c->storage, c->has_solid, c->target_blocks,
+                       c->march_rows, c->march_hold, flags,      c->psi_polls};
   put(ints, sizeof ints);
   put(&c->geo, sizeof c->geo);
   put(&c->p, sizeof c->p);

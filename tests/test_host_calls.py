@@ -1,0 +1,74 @@
+"""The runtime calls that the library's host code makes, on a stand-in for the
+HIP runtime (fake_hip.cpp: host memory, kernels counted and not run).  Each test
+runs its lines in a process of its own, where the stand-in is loaded first.
+
+In those lines: D the package, hip the stand-in, calls(name) and launches(part)
+its counts, lattice() a lattice with parameters and populations."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PREAMBLE = """
+import ctypes, sys
+import numpy as np
+hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+for fn in ("calls", "launches", "live"):
+    getattr(hip, "fake_hip_" + fn).restype = ctypes.c_int64
+sys.path.insert(0, sys.argv[2])
+import dlbc_amd as D
+
+def calls(name):
+    return hip.fake_hip_calls(name.encode())
+
+def launches(part):
+    return hip.fake_hip_launches(part.encode())
+
+def live(device):
+    return hip.fake_hip_live(device)
+
+def fail(name, nth=1, code=1):
+    hip.fake_hip_fail(name.encode(), nth, code)
+
+def lattice(n, nc=2, sc=True, storage="f64", device=0):
+    d, q = len(n), (19 if len(n) == 3 else 9)
+    lat = D.Lattice(d, q, nc, n, storage=storage, device=device)
+    lat.set_params([1.0] * nc, [[0.0 if i == j else 3.6 for j in range(nc)] for i in range(nc)],
+                   None, None, None, "BDist2", "Exponential", sc)
+    for f in range(nc):
+        lat.init_fluid(f, "EqDist", [0.5], "BDist2")
+    return lat
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-fPIC", "-shared", "-pthread",
+                    os.path.join(HERE, "fake_hip.cpp"), "-o", so], check=True)
+
+    def go(lines):
+        r = subprocess.run([sys.executable, "-c", PREAMBLE + textwrap.dedent(lines), so,
+                            os.path.dirname(HERE)], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return go
+
+
+@pytest.mark.parametrize("n,nc,sc,steps", [((64, 64), 2, True, 33), ((64, 64), 1, False, 200),
+                                           ((20, 20, 20), 2, True, 33), ((20, 20, 20), 1, False, 35),
+                                           ((70, 80, 64), 2, True, 33)], ids=str)
+def test_a_lattice_keeps_a_graph_of_each_buffer_parity(run, n, nc, sc, steps):
+    run(f"""
+    lat = lattice({n}, {nc}, {sc})
+    for k in range(8):
+        lat.step({steps}, graph=True)
+    assert calls("hipGraphInstantiate") == 2, calls("hipGraphInstantiate")
+    assert calls("hipGraphLaunch") == 8 * ({steps} // 32)
+    lat.set_launch(512)  # new arguments: captured again
+    lat.step(32, graph=True)
+    assert calls("hipGraphInstantiate") == 3
+    """)
