@@ -1978,8 +1978,10 @@ struct dlbc_batch {
   int nflag = 0, psi_set = 0;
   bool one_launch_off = false;  // no memory for them
   bool items_dirty = true;
-  hipGraphExec_t graph = nullptr;
-  int graph_sig = -1;  // batch_launch_sig() when the graph was captured
+  // two captured steps for each flag set that a call starts with, and the
+  // batch_launch_sig() that they were captured under
+  hipGraphExec_t graph[2] = {nullptr, nullptr};
+  int graph_sig = -1;
   std::string err;
 };
 
@@ -2003,10 +2005,12 @@ int bfail(dlbc_batch *b, int code, const char *fmt, ...) {
   } while (0)
 
 void batch_drop_graph(dlbc_batch *b) {
-  if (!b->graph) return;
+  if (!b->graph[0] && !b->graph[1]) return;
   if (b->stream) (void)hipStreamSynchronize(b->stream);  // replays may be in flight
-  (void)hipGraphExecDestroy(b->graph);
-  b->graph = nullptr;
+  for (auto &g : b->graph) {
+    if (g) (void)hipGraphExecDestroy(g);
+    g = nullptr;
+  }
 }
 
 // Work list for the current tile height and chunk length, on the device.
@@ -2060,11 +2064,11 @@ bool batch_one_launch(const dlbc_batch *b) {
 
 // The host state that picks kernels at launch beyond the configuration: any
 // member with solids (the kernels' SOLID variants) and any with Shan-Chen (the
-// split schedule's psi pass), one launch or two and the flags it starts with.
-// A captured graph is only valid for the value it was captured with.
+// split schedule's psi pass), one launch or two.  A captured graph is only valid
+// for the value it was captured with, and for the flag set it is kept under.
 int batch_launch_sig(const dlbc_batch *b) {
   return (batch_has_solid(b) ? 1 : 0) | (batch_has_sc(b, 0, (int)b->ctx.size()) ? 2 : 0) |
-         (batch_one_launch(b) ? 4 + 8 * b->psi_set : 0);
+         (batch_one_launch(b) ? 4 : 0);
 }
 
 // The turns and flags of that launch, once per batch; without the memory for
@@ -2138,7 +2142,7 @@ int batch_prepare(dlbc_batch *b) {
   }
   const int rs = batch_split_ready(b);
   if (rs) return rs;
-  if (b->graph && b->graph_sig != batch_launch_sig(b)) batch_drop_graph(b);
+  if (b->graph_sig != batch_launch_sig(b)) batch_drop_graph(b);
   if (b->items_dirty) return batch_build_items(b);
   return DLBC_OK;
 }
@@ -2323,7 +2327,10 @@ int dlbc_batch_step(dlbc_batch *b, int nsteps, int use_graph) {
   // the persistent split launch is cooperative and is not captured: one
   // launch per step either way
   if (use_graph && nsteps >= 2 && b->kernel != 3) {
-    if (!b->graph) {  // two steps: even parity, then odd
+    // (an odd step count leaves the other flag set to the next call; the set of
+    // a batch that does not take one launch stands still)
+    hipGraphExec_t &graph = b->graph[b->psi_set];
+    if (!graph) {  // two steps: even parity, then odd
       hipGraph_t g = nullptr;
       BHIPCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
       int rc0 = batch_launch(b, b->d_items, nit, 0, b->grid);
@@ -2334,12 +2341,13 @@ int dlbc_batch_step(dlbc_batch *b, int nsteps, int use_graph) {
         return rc1;
       }
       BHIPCHK(b, ec);
-      const hipError_t ei = hipGraphInstantiate(&b->graph, g, nullptr, nullptr, 0);
+      const hipError_t ei = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
       (void)hipGraphDestroy(g);
+      if (ei != hipSuccess) graph = nullptr;
       BHIPCHK(b, ei);
       b->graph_sig = batch_launch_sig(b);
     }
-    for (; t + 2 <= nsteps; t += 2) BHIPCHK(b, hipGraphLaunch(b->graph, b->stream));
+    for (; t + 2 <= nsteps; t += 2) BHIPCHK(b, hipGraphLaunch(graph, b->stream));
   }
   for (; t < nsteps; ++t) {
     rc = batch_launch(b, b->d_items, nit, t & 1, b->grid);

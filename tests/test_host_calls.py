@@ -72,3 +72,24 @@ def test_a_lattice_keeps_a_graph_of_each_buffer_parity(run, n, nc, sc, steps):
     lat.step(32, graph=True)
     assert calls("hipGraphInstantiate") == 3
     """)
+
+
+@pytest.mark.parametrize("n,steps", [((120, 120, 120), 3), ((120, 120, 120), 4), ((16, 16, 16), 3)],
+                         ids=str)
+def test_a_batch_keeps_a_graph_of_each_flag_set(run, n, steps):
+    run(f"""
+    lats = [lattice({n}, storage="f32_shift") for _ in range(2)]
+    batch = D.Batch(lats)
+    batch.set_config(8, 64, 512, 2)
+    for k in range(8):
+        batch.step({steps}, graph=True)
+    one = {n} == (120, 120, 120)  # one launch per step: flags in two sets
+    assert launches("psi") == (0 if one else {steps} % 2 * 8 + 2), launches("psi")
+    assert calls("hipGraphInstantiate") == (2 if one and {steps} % 2 else 1)
+    assert calls("hipGraphLaunch") == 8 * ({steps} // 2)
+    lats[0].set_params([1.0, 1.0], None, None, None, None, "BDist2", "Exponential", False)
+    lats[1].set_params([1.0, 1.0], None, None, None, None, "BDist2", "Exponential", False)
+    made = calls("hipGraphInstantiate")
+    batch.step(2, graph=True)  # other kernels: captured again
+    assert calls("hipGraphInstantiate") == made + 1
+    """)
