@@ -584,13 +584,14 @@ int order_strip(int storage) {
 // 190x151x117 with solids 292 / 249, 256^3 1390 / 1120; FP16 without solids
 // 128^3 91 / 90, 256^3 719 / 657, 384^3 2570 / 2310.  FP16 with solids, whose
 // collide is bound by its instructions and whose psi then runs at the collide's
-// four waves per SIMD, 836 / 943 at 256^3: two launches.
+// four waves per SIMD, 836 / 943 at 256^3: two launches.  Lattices of thin planes
+// or very long rows keep two launches, too (split_order_serves).
 bool split_one_launch(const dlbc_gpu_ctx *c) {
   if (c->d != 3 || c->C != 2 || !c->p.sc || c->geo.order_chunk != 0 || c->one_launch_off)
     return false;
   if (c->storage == DLBC_STORAGE_F16_SHIFT && c->has_solid) return false;
   const int64_t blocks = c->storage == DLBC_STORAGE_F64 ? 2500 : 6000;
-  return c->geo.sites >= blocks * split_sites(c);
+  return c->geo.sites >= blocks * split_sites(c) && split_order_serves(c->geo, split_sites(c));
 }
 
 // Whether a step is one launch over small tiles (kernels_tile.hpp): D2Q9 with
@@ -2055,11 +2056,14 @@ bool batch_has_sc(const dlbc_batch *b, int l0, int l1) {
 }
 
 // Whether the split pair of the whole batch is one launch (the rule of
-// split_one_launch).
+// split_one_launch, for every member).
 bool batch_one_launch(const dlbc_batch *b) {
   if (b->one_launch_off || !batch_has_sc(b, 0, (int)b->ctx.size())) return false;
   if (b->storage == DLBC_STORAGE_F16_SHIFT && batch_has_solid(b)) return false;
-  return b->h_first.back() >= 6000;
+  if (b->h_first.back() < 6000) return false;
+  for (auto *c : b->ctx)
+    if (!split_order_serves(c->geo, kShiftSites)) return false;
+  return true;
 }
 
 // The host state that picks kernels at launch beyond the configuration: any

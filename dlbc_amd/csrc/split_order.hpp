@@ -99,6 +99,23 @@ __host__ __device__ inline void split_needs(const Geo &g, int SB, int blk, int k
   hi = (x * plane + r1 * g.nz + g.nz - 1) / SB;
 }
 
+// Whether a lattice is served by this order: a collide wave looks at the flags of
+// every block in split_needs, and the psi of all of them stands in front of it.
+// Both are few where a block meets no more than two planes (planes of a block's
+// sites or more; a block over more planes would wait for the whole lattice) and
+// rows are not too long, of which a collide waits for nine whole ones.  us per
+// step, two launches / one: FP64 rows of 16, 128, 256 and 512 blocks (16 x 16
+// rows) 361 / 314, 715 / 656, 1442 / 1441 and 2936 / 3128; FP32 rows of 128, 256
+// and 512 blocks 715 / 636, 1426 / 1384 and 366 / 390; planes of one block
+// (16384 x 8 x 16) FP64 347 / 290, FP32 (8192 x 16 x 16) 173 / 153.  A lattice of
+// no more than kOrderRowBlocks blocks (a member of a batch) has no more to wait
+// for than such a row.
+constexpr int kOrderRowBlocks = 256;
+inline bool split_order_serves(const Geo &g, int SB) {
+  const int64_t most = (int64_t)kOrderRowBlocks * SB;
+  return g.sites <= most || ((int64_t)g.ny * g.nz >= SB && g.nz <= most);
+}
+
 // The psi blocks and the collide blocks of a lattice in the order of their
 // visits, numbered from blk0, appended to psi and col; need: for every collide
 // the psi places it wants in front of it, counted in the whole of psi.

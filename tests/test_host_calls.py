@@ -93,3 +93,28 @@ def test_a_batch_keeps_a_graph_of_each_flag_set(run, n, steps):
     batch.step(2, graph=True)  # other kernels: captured again
     assert calls("hipGraphInstantiate") == made + 1
     """)
+
+
+@pytest.mark.parametrize("storage,n,one", [
+    ("f64", (100000, 10, 10), False), ("f64", (20000, 4, 4), False), ("f64", (4, 4, 65536), False),
+    ("f64", (16384, 8, 16), True), ("f64", (2, 5, 32768), True), ("f64", (128, 4, 4096), True),
+    ("f32_shift", (7000, 15, 16), False), ("f32_shift", (5, 5, 65537), False),
+    ("f32_shift", (8192, 16, 16), True), ("f32_shift", (5, 5, 65536), True),
+    ("f16_shift", (100000, 10, 10), False), ("f16_shift", (8192, 16, 16), True)], ids=str)
+def test_thin_planes_and_long_rows_take_two_launches(run, storage, n, one):
+    """A block of sites that meets more than two planes would wait for the whole
+    lattice, and long rows for many blocks."""
+    run(f"""
+    lat = lattice({n}, storage="{storage}")
+    lat.step(3)
+    assert launches("split_psi") == {0 if one else 3}, launches("split_psi")
+    assert launches("split_collide") == 3
+    if "{storage}" != "f64":
+        # a large member of this shape decides for its batch, a small one does not
+        for other in ((128, 128, 96), (1000, 4, 4)):
+            batch = D.Batch([lattice(other, storage="{storage}"), lat])
+            batch.set_config(8, 64, 512, 2)
+            psi = launches("batch_split_psi")
+            batch.step(3)
+            assert launches("batch_split_psi") - psi == {0 if one else 3}
+    """)

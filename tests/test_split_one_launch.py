@@ -110,3 +110,19 @@ def test_batch_in_one_launch_equals_lattices_alone(D, storage, solid):
         batch.synchronize()
     for a, b, n in zip(alone, members, sizes):
         _same(a, b, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,kernels", [((21000, 4, 4), 2), ((5, 2, 32769), 2), ((2600, 8, 16), 1),
+                                       ((5, 2, 32768), 1)], ids=str)
+def test_thin_planes_and_long_rows_equal_oracle(D, n, kernels):
+    """Planes of fewer sites than a block and rows of more than 256 blocks take
+    two launches; planes of one block and rows of 256 are the smallest and the
+    longest that take one."""
+    from oracle.oracle import Oracle
+    p = _params(n, "BDist2", False)
+    g, o = D.Lattice.from_params(p, schedule="split"), Oracle.from_params(p)
+    assert len(g.step_timed(2)[1]) == kernels
+    g.step(1)
+    o.run(3)
+    _same(g, o, n)
