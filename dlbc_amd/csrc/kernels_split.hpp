@@ -102,13 +102,43 @@ __device__ inline bool split_lane(const Geo &g, int blk, int w, int &s, int &f) 
 // ---- both passes in one launch -------------------------------------------------
 // Every block of sites is visited by a psi workgroup and later by a collide
 // workgroup, in the order of a table (split_order.hpp).  psi goes from one to
-// the other through S (P): written through the L2 of the XCD that made it, and
-// then a flag for its block.  A collide wave looks at the flags of the blocks
-// that it reads before it reads them; until then no line of theirs is in its
-// L2, and a line is written by one wave with one store, so that no line is read
-// half written.
-// A wave that finds no flags for too long computes that psi itself (the same
-// values): no wave waits for one that has not started.
+// the other through S (P), and then a flag for its block; a collide wave looks
+// at the flags of the blocks that it reads before it reads them.  A wave that
+// finds no flags for too long computes that psi itself (the same values): no
+// wave waits for one that has not started.
+//
+// The hand-over has no release or acquire of the language: those are fences of
+// whole caches at agent scope (buffer_wbl2, buffer_inv), and an acquire in every
+// collide wave alone costs more than the launch saves (steps of FP64 128^3
+// 1.95 times as long, 256^3 1.86, FP32 190x151x117 1.77, FP16 384^3 2.97; a
+// release in every psi wave takes longer still).  It is made for gfx950 and rests
+// on this:
+//  - Out: psi and flags are stored at agent scope, which writes through the L2 of
+//    the XCD to what all XCDs share, and such a store leaves vmcnt when it is
+//    there.  Every psi wave waits for vmcnt 0, then the workgroup's barrier, then
+//    one lane stores the flag.
+//  - In: flags are loaded at agent scope, past the XCD's own caches.  psi is
+//    loaded only after the flags were seen (a branch on their value, and a
+//    barrier to the compiler), by ordinary loads; those are right as long as
+//    neither L1 nor L2 of the reader holds an older copy of the line:
+//     * a launch starts with both invalidated (S and P were written on other XCDs
+//       by the launch before, like the populations, which rely on it, too);
+//     * in the launch no line is read before its flag: a collide reads psi only
+//       in split_needs, psi workgroups read none, and caches fetch only lines
+//       that are asked for;
+//     * a line belongs to one wave: 64 sites of one component are whole lines of
+//       128 bytes, as blocks and the components' strides are whole multiples of 64
+//       sites (asserted below, and in split_order_serves).  Its other bytes are
+//       densities of solid sites, which no launch writes.
+//  - A wave that computes psi itself stores the values that the others store, and
+//    reads them after vmcnt 0 through its own XCD's L2, which they went through.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "the hand-over of psi is made for the caches of gfx950"
+#endif
+static_assert(kSplitThreads / 2 % 64 == 0 && kShiftSites % 64 == 0 &&
+                  64 * sizeof(double) % 128 == 0 && 64 * sizeof(float) % 128 == 0,
+              "a wave writes whole lines of psi");
+
 struct SplitPlan {
   const int32_t *order;  // what each turn of eight workgroups does
   uint8_t *flags;        // [2][nflag]: the psi of a block is written

@@ -109,10 +109,12 @@ __host__ __device__ inline void split_needs(const Geo &g, int SB, int blk, int k
 // and 512 blocks 715 / 636, 1426 / 1384 and 366 / 390; planes of one block
 // (16384 x 8 x 16) FP64 347 / 290, FP32 (8192 x 16 x 16) 173 / 153.  A lattice of
 // no more than kOrderRowBlocks blocks (a member of a batch) has no more to wait
-// for than such a row.
+// for than such a row.  (Components of whole tiles of 64 sites: no line of psi
+// holds sites of two waves.)
 constexpr int kOrderRowBlocks = 256;
 inline bool split_order_serves(const Geo &g, int SB) {
   const int64_t most = (int64_t)kOrderRowBlocks * SB;
+  if (g.sp % 64 != 0) return false;
   return g.sites <= most || ((int64_t)g.ny * g.nz >= SB && g.nz <= most);
 }
 
