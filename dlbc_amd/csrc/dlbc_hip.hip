@@ -109,7 +109,8 @@ int ensure_scratch(dlbc_gpu_ctx *c, size_t bytes) {
     c->scratch = nullptr;
     c->scratch_bytes = 0;
   }
-  if (hipMalloc(&c->scratch, bytes) != hipSuccess)
+  const OnDevice on(c->device);
+  if (!on.ok || hipMalloc(&c->scratch, bytes) != hipSuccess)
     return fail(c, DLBC_ERR_NOMEM, "cannot allocate %zu bytes of device scratch", bytes);
   c->scratch_bytes = bytes;
   c->dev_bytes += (int64_t)bytes;
@@ -444,6 +445,7 @@ int shifted_self_ready(dlbc_gpu_ctx *c) {
     batch_items(&c->geo, 1, 8, chunk, items);
     if (c->d_items) HIPCHK(c, hipFree(c->d_items));
     c->d_items = nullptr;
+    const OnDevice on(c->device);
     HIPCHK(c, hipMalloc(&c->d_items, sizeof(BatchItem) * items.size()));
     HIPCHK(c, hipMemcpyAsync(c->d_items, items.data(), sizeof(BatchItem) * items.size(),
                              hipMemcpyHostToDevice, c->stream));
@@ -626,7 +628,9 @@ int split_ready(dlbc_gpu_ctx *c) {
   const size_t ob = sizeof(int32_t) * o.size();
   int32_t *d = nullptr;
   uint8_t *fl = nullptr;
-  if (hipMalloc(&d, ob) != hipSuccess || hipMalloc(&fl, 2 * (size_t)nflag) != hipSuccess) {
+  const OnDevice on(c->device);
+  if (!on.ok || hipMalloc(&d, ob) != hipSuccess ||
+      hipMalloc(&fl, 2 * (size_t)nflag) != hipSuccess) {
     (void)hipGetLastError();
     if (d) (void)hipFree(d);
     c->one_launch_off = true;
@@ -2032,6 +2036,7 @@ int batch_build_items(dlbc_batch *b) {
   if (b->h_items.size() > b->items_cap) {
     if (b->d_items) BHIPCHK(b, hipFree(b->d_items));
     b->d_items = nullptr;
+    const OnDevice on(b->device);
     BHIPCHK(b, hipMalloc(&b->d_items, sizeof(BatchItem) * b->h_items.size()));
     b->items_cap = b->h_items.size();
   }
@@ -2098,7 +2103,9 @@ int batch_split_ready(dlbc_batch *b) {
   const size_t ob = sizeof(int32_t) * turns.size();
   int32_t *d = nullptr;
   uint8_t *fl = nullptr;
-  if (hipMalloc(&d, ob) != hipSuccess || hipMalloc(&fl, 2 * (size_t)nflag) != hipSuccess) {
+  const OnDevice on(b->device);
+  if (!on.ok || hipMalloc(&d, ob) != hipSuccess ||
+      hipMalloc(&fl, 2 * (size_t)nflag) != hipSuccess) {
     (void)hipGetLastError();
     if (d) (void)hipFree(d);
     b->one_launch_off = true;

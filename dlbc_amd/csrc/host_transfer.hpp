@@ -29,6 +29,25 @@ namespace dlbc {
 constexpr size_t kSlotBytes = 2u << 20;
 constexpr int kTransferThreads = 8, kTransferKept = 16;
 
+// `device` is the calling thread's current one while this lives (ok: it is).
+struct OnDevice {
+  int before = -1;
+  bool ok = true;
+  explicit OnDevice(int device) {
+    if (hipGetDevice(&before) != hipSuccess) before = -1;
+    if (before == device)
+      before = -1;  // nothing to give back
+    else
+      ok = hipSetDevice(device) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+  }
+  ~OnDevice() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+  OnDevice(const OnDevice &) = delete;
+  OnDevice &operator=(const OnDevice &) = delete;
+};
+
 struct PinnedSlot {
   void *p = nullptr;
   hipEvent_t done = nullptr;
@@ -55,8 +74,7 @@ struct SlotPool {
     for (auto &s : idle) drop(s);
     idle.clear();
   }
-  // A slot for `device` (the calling thread's current one); p is null where
-  // there is no memory.
+  // A slot for `device`; p is null where there is no memory.
   PinnedSlot take(int device) {
     {
       std::lock_guard<std::mutex> lock(mu);
@@ -69,7 +87,8 @@ struct SlotPool {
     }
     PinnedSlot s;
     s.device = device;
-    if (hipHostMalloc(&s.p, kSlotBytes, hipHostMallocPortable) != hipSuccess ||
+    const OnDevice on(device);
+    if (!on.ok || hipHostMalloc(&s.p, kSlotBytes, hipHostMallocPortable) != hipSuccess ||
         hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess) {
       (void)hipGetLastError();
       drop(s);

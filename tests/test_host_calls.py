@@ -118,3 +118,42 @@ def test_thin_planes_and_long_rows_take_two_launches(run, storage, n, one):
             batch.step(3)
             assert launches("batch_split_psi") - psi == {0 if one else 3}
     """)
+
+
+@pytest.mark.parametrize("current", [0, 1])
+def test_memory_is_made_on_the_device_of_its_lattice(run, current):
+    """What is allocated after the creation of a lattice or a batch lies on its
+    device, whichever the calling thread has current, and that one stays."""
+    run(f"""
+    lats = [lattice((70, 80, 64), device=k) for k in range(2)]
+    shifted = [lattice((128, 128, 96), storage="f32_shift", device=k) for k in range(2)]
+    tiled = [lattice((16, 16, 16), storage="f32_shift", device=k) for k in range(2)]
+    batches = [D.Batch([lat]) for lat in shifted]
+    for b in batches:
+        b.set_config(8, 64, 512, 2)
+    hip.hipSetDevice({current})
+    now = ctypes.c_int(-1)
+
+    def lies_on(device, work, count):
+        before = live(device), live(1 - device)
+        work()
+        assert (live(device) - before[0], live(1 - device) - before[1]) == (count, 0), (
+            device, live(device) - before[0], live(1 - device) - before[1])
+        hip.hipGetDevice(ctypes.byref(now))
+        assert now.value == {current}
+
+    for k in (0, 1):
+        lies_on(k, lambda: lats[k].step(1), 2)  # order and flags
+        lies_on(k, lambda: batches[k].step(1), 3)  # and the batch's items
+        lies_on(k, lambda: lats[k].step(1), 0)
+        tiled[k].set_schedule("fused")
+        lies_on(k, lambda: tiled[k].step(1), 1)  # its items
+        lies_on(k, lambda: tiled[k].density(0), 2)  # a slot: its memory and event
+        before = live(1 - k)
+        lats[k].density(0)  # scratch, and slots as the threads take them
+        assert live(1 - k) == before
+    del lats, shifted, tiled, batches, b
+    import gc
+    gc.collect()
+    assert live(0) == 0 and live(1) == 0
+    """)
