@@ -53,6 +53,7 @@ struct dlbc_gpu_ctx {
   uint8_t *psi_flags = nullptr;
   int nflag = 0, psi_set = 0, psi_polls = kPsiPolls;
   bool one_launch_off = false;  // no memory for them
+  bool flags_unknown = false;   // a call failed: which flags are up is not known
   int has_solid = 0;
   bool params_set = false, pops_uploaded[kMaxC] = {false, false, false, false};
   bool solid_rho_dirty = true;
@@ -93,11 +94,14 @@ int fail(dlbc_gpu_ctx *c, int code, const char *fmt, ...) {
   return code;
 }
 
+// (The error is reported here and not by the next call's hipGetLastError.)
 #define HIPCHK(ctx, call)                                                                   \
   do {                                                                                      \
     hipError_t e_ = (call);                                                                 \
-    if (e_ != hipSuccess)                                                                   \
+    if (e_ != hipSuccess) {                                                                 \
+      (void)hipGetLastError();                                                              \
       return fail((ctx), DLBC_ERR_HIP, "%s failed: %s", #call, hipGetErrorString(e_));      \
+    }                                                                                       \
   } while (0)
 
 int ensure_scratch(dlbc_gpu_ctx *c, size_t bytes) {
@@ -611,9 +615,32 @@ bool tile_step(const dlbc_gpu_ctx *c) {
   return c->C > 2 || c->geo.sites <= 160000 || c->geo.sites >= 1500000;
 }
 
+// While a call launches steps, and until it has done so without an error, the
+// flags of the one-launch step (of a context or a batch) count as unknown: a
+// launch that did not run leaves the set of the next one up.
+template <class Owner>
+struct StepsGuard {
+  Owner *o;
+  explicit StepsGuard(Owner *owner) : o(owner) { o->flags_unknown = true; }
+  int done(int rc) {
+    if (rc == DLBC_OK) o->flags_unknown = false;
+    return rc;
+  }
+};
+
+// Takes all flags down (in the stream's order) if they are not known.
+template <class Owner>
+hipError_t flags_ready(Owner *o) {
+  if (!o->flags_unknown || !o->psi_flags) return hipSuccess;
+  const hipError_t e = hipMemsetAsync(o->psi_flags, 0, 2 * (size_t)o->nflag, o->stream);
+  if (e == hipSuccess) o->psi_set = 0;
+  return e;
+}
+
 // The order and the flags of that launch, once per context.  Without the memory
 // for them the step stays at two launches.
 int split_ready(dlbc_gpu_ctx *c) {
+  HIPCHK(c, flags_ready(c));
   if (c->order || effective_schedule(c) != DLBC_SCHED_SPLIT || tile_step(c) ||
       !split_one_launch(c))
     return DLBC_OK;
@@ -675,6 +702,7 @@ struct SplitStep {
       };
       if (split_one_launch(c)) {
         pass(2);
+        HIPCHK(c, hipGetLastError());
         c->psi_set ^= 1;
       } else {
         if (c->p.sc) pass(0);
@@ -812,10 +840,11 @@ int do_steps(dlbc_gpu_ctx *c, int nsteps, Timer *tm) {
   int rc = prepare(c);
   if (!rc) rc = split_ready(c);
   if (rc) return rc;
+  StepsGuard<dlbc_gpu_ctx> steps(c);
   rc = advance(c, effective_schedule(c), nsteps, tm);
   if (rc) return rc;
   HIPCHK(c, hipGetLastError());
-  return DLBC_OK;
+  return steps.done(DLBC_OK);
 }
 
 // Replays may still be in flight on the stream: wait for them before the
@@ -1604,6 +1633,7 @@ int dlbc_gpu_step_graph(dlbc_gpu_ctx *c, int nsteps) {
     c->graph_key.swap(key);
   }
   Timer tm{c, false};
+  StepsGuard<dlbc_gpu_ctx> steps(c);
   int t = 0;
   if (nsteps >= kGraphSteps) {
     const int par = c->popA == c->bufX ? 0 : 1;
@@ -1612,14 +1642,16 @@ int dlbc_gpu_step_graph(dlbc_gpu_ctx *c, int nsteps) {
       hipGraph_t g = nullptr;
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
       const int rcc = advance(c, sched, kGraphSteps, &tm);
+      const hipError_t el = hipGetLastError();  // of the launches
       const hipError_t ec = hipStreamEndCapture(c->stream, &g);
       c->popA = a;  // captured, not run
       c->popB = b;
-      if (rcc) {
+      if (rcc || el != hipSuccess || ec != hipSuccess) {
         if (g) (void)hipGraphDestroy(g);
-        return rcc;
+        if (rcc) return rcc;
+        HIPCHK(c, el);
+        HIPCHK(c, ec);
       }
-      HIPCHK(c, ec);
       const hipError_t ei = hipGraphInstantiate(&c->graph[par], g, nullptr, nullptr, 0);
       (void)hipGraphDestroy(g);
       if (ei != hipSuccess) c->graph[par] = nullptr;
@@ -1631,7 +1663,7 @@ int dlbc_gpu_step_graph(dlbc_gpu_ctx *c, int nsteps) {
   rc = advance(c, sched, nsteps - t, &tm);
   if (rc) return rc;
   HIPCHK(c, hipGetLastError());
-  return DLBC_OK;
+  return steps.done(DLBC_OK);
 }
 
 int dlbc_gpu_advect(dlbc_gpu_ctx *c) {
@@ -1982,6 +2014,7 @@ struct dlbc_batch {
   uint8_t *psi_flags = nullptr;
   int nflag = 0, psi_set = 0;
   bool one_launch_off = false;  // no memory for them
+  bool flags_unknown = false;   // (as of a context)
   bool items_dirty = true;
   // two captured steps for each flag set that a call starts with, and the
   // batch_launch_sig() that they were captured under
@@ -2005,8 +2038,10 @@ int bfail(dlbc_batch *b, int code, const char *fmt, ...) {
 #define BHIPCHK(b, call)                                                                    \
   do {                                                                                      \
     hipError_t e_ = (call);                                                                 \
-    if (e_ != hipSuccess)                                                                   \
+    if (e_ != hipSuccess) {                                                                 \
+      (void)hipGetLastError();                                                              \
       return bfail((b), DLBC_ERR_HIP, "%s failed: %s", #call, hipGetErrorString(e_));       \
+    }                                                                                       \
   } while (0)
 
 void batch_drop_graph(dlbc_batch *b) {
@@ -2083,6 +2118,7 @@ int batch_launch_sig(const dlbc_batch *b) {
 // The turns and flags of that launch, once per batch; without the memory for
 // them the batch stays at two launches.
 int batch_split_ready(dlbc_batch *b) {
+  BHIPCHK(b, flags_ready(b));
   if (b->order || b->kernel != 2 || !batch_one_launch(b)) return DLBC_OK;
   std::vector<int32_t> turns;
   try {
@@ -2334,6 +2370,7 @@ int dlbc_batch_step(dlbc_batch *b, int nsteps, int use_graph) {
   int rc = batch_prepare(b);
   if (rc) return rc;
   const int nit = (int)b->h_items.size();
+  StepsGuard<dlbc_batch> steps(b);
   int t = 0;
   // the persistent split launch is cooperative and is not captured: one
   // launch per step either way
@@ -2364,7 +2401,7 @@ int dlbc_batch_step(dlbc_batch *b, int nsteps, int use_graph) {
     rc = batch_launch(b, b->d_items, nit, t & 1, b->grid);
     if (rc) return rc;
   }
-  return batch_finish(b, nsteps);
+  return steps.done(batch_finish(b, nsteps));
 }
 
 int dlbc_batch_step_looped(dlbc_batch *b, int nsteps) {
@@ -2372,6 +2409,7 @@ int dlbc_batch_step_looped(dlbc_batch *b, int nsteps) {
   if (nsteps == 0) return DLBC_OK;
   int rc = batch_prepare(b);
   if (rc) return rc;
+  StepsGuard<dlbc_batch> steps(b);
   for (int t = 0; t < nsteps; ++t)
     for (size_t l = 0; l + 1 < b->lat_first.size(); ++l) {
       const int first = b->lat_first[l], cnt = b->lat_first[l + 1] - first;
@@ -2380,13 +2418,14 @@ int dlbc_batch_step_looped(dlbc_batch *b, int nsteps) {
                                          std::min(b->grid, (cnt + 7) / 8 * 8));
       if (rc) return rc;
     }
-  return batch_finish(b, nsteps);
+  return steps.done(batch_finish(b, nsteps));
 }
 
 int dlbc_batch_autotune(dlbc_batch *b, int *out, double *best_ms) {
   if (!b) return DLBC_ERR_ARG;
   int rc = batch_prepare(b);
   if (rc) return rc;
+  StepsGuard<dlbc_batch> steps(b);
   const int tys[2] = {8, 4};
   const int chunks[4] = {16, 32, 64, 1 << 20};
   const int grids[4] = {256, 512, 1024, 2048};
@@ -2456,7 +2495,7 @@ int dlbc_batch_autotune(dlbc_batch *b, int *out, double *best_ms) {
     out[3] = bk;
   }
   if (best_ms) *best_ms = best;
-  return DLBC_OK;
+  return steps.done(DLBC_OK);
 }
 
 int dlbc_batch_synchronize(dlbc_batch *b) {

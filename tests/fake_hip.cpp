@@ -3,8 +3,9 @@
 //
 // Loaded with RTLD_GLOBAL before the library, its functions take the place of
 // the runtime's.  Memory is the host's and copies are made at once; a kernel
-// launch is counted under the kernel's (mangled) name and does nothing.  Calls
-// are counted, can be made to fail, and remember the device that was current.
+// launch is counted under the kernel's (mangled) name and does nothing but what
+// the one-launch step does to its flags.  Calls are counted, can be made to fail,
+// and remember the device that was current.
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -59,6 +60,36 @@ int gone(void *p) {
   return 0;
 }
 
+// The flags of the one-launch step (SplitPlan, the seventh argument of its
+// kernels): all of a launch's own set are down when it starts and up when it has
+// ended, and those of the other set are down then.
+struct Plan {
+  const int32_t *order;
+  uint8_t *flags;
+  int nflag, set, polls;
+};
+int64_t flags_up = 0;  // launches that started with some of their flags up
+void run_plan(const Plan &q) {
+  uint8_t *own = q.flags + (int64_t)q.set * q.nflag, *other = q.flags + (int64_t)(q.set ^ 1) * q.nflag;
+  for (int k = 0; k < q.nflag; ++k)
+    if (own[k]) {
+      ++flags_up;
+      break;
+    }
+  std::memset(own, 1, q.nflag);
+  std::memset(other, 0, q.nflag);
+}
+bool one_launch(const std::string &name) {  // the last template argument: true
+  return name.find("split_collide") != std::string::npos &&
+         name.find("Lb1EEEv") != std::string::npos;
+}
+struct Graph {
+  std::vector<Plan> plans;
+  int64_t nodes = 0;
+};
+std::map<void *, Graph> capturing;  // by stream
+int64_t graph_nodes = 0;            // kernels of the graph launched last
+
 struct Dim3 {
   uint32_t x, y, z;
 };
@@ -91,6 +122,15 @@ int64_t fake_hip_live(int device) {
   std::lock_guard<std::mutex> lock(mu);
   return live[device];
 }
+// Launches of the one-launch step that started with some of their flags up.
+int64_t fake_hip_flags_up() {
+  std::lock_guard<std::mutex> lock(mu);
+  return flags_up;
+}
+int64_t fake_hip_graph_nodes() {
+  std::lock_guard<std::mutex> lock(mu);
+  return graph_nodes;
+}
 // The nth call of `name` from now on returns `code`.
 void fake_hip_fail(const char *name, int nth, int code) {
   std::lock_guard<std::mutex> lock(mu);
@@ -122,10 +162,20 @@ int __hipPopCallConfiguration(Dim3 *grid, Dim3 *block, size_t *shared, void **st
   *stream = c.stream;
   return 0;
 }
-int hipLaunchKernel(const void *host, Dim3, Dim3, void **, size_t, void *) {
+int hipLaunchKernel(const void *host, Dim3, Dim3, void **args, size_t, void *stream) {
   if (const int e = called("hipLaunchKernel")) return e;
   std::lock_guard<std::mutex> lock(mu);
-  ++launches[kernels[host]];
+  const std::string &name = kernels[host];
+  ++launches[name];
+  const auto c = capturing.find(stream);
+  if (c != capturing.end()) ++c->second.nodes;
+  if (one_launch(name)) {
+    const Plan q = *static_cast<const Plan *>(args[6]);
+    if (c != capturing.end())
+      c->second.plans.push_back(q);
+    else
+      run_plan(q);
+  }
   return 0;
 }
 int hipLaunchCooperativeKernel(const void *host, Dim3 grid, Dim3 block, void **args,
@@ -220,27 +270,40 @@ int hipEventElapsedTime(float *ms, void *, void *) {
   *ms = 1.0f;
   return 0;
 }
-int hipStreamBeginCapture(void *, int) { return called("hipStreamBeginCapture"); }
-int hipStreamEndCapture(void *, void **g) {
-  *g = nullptr;
-  if (const int e = called("hipStreamEndCapture")) return e;
-  *g = std::calloc(1, 8);
+int hipStreamBeginCapture(void *stream, int) {
+  if (const int e = called("hipStreamBeginCapture")) return e;
+  std::lock_guard<std::mutex> lock(mu);
+  capturing[stream] = Graph{};
   return 0;
 }
-int hipGraphInstantiate(void **x, void *, void *, char *, size_t) {
+int hipStreamEndCapture(void *stream, void **g) {
+  *g = nullptr;
+  const int e = called("hipStreamEndCapture");
+  std::lock_guard<std::mutex> lock(mu);
+  if (!e) *g = new Graph(capturing[stream]);
+  capturing.erase(stream);
+  return e;
+}
+int hipGraphInstantiate(void **x, void *g, void *, char *, size_t) {
   *x = nullptr;
   if (const int e = called("hipGraphInstantiate")) return e;
-  *x = std::calloc(1, 8);
+  *x = new Graph(*static_cast<Graph *>(g));
   return 0;
 }
 int hipGraphDestroy(void *g) {
-  std::free(g);
+  delete static_cast<Graph *>(g);
   return 0;
 }
 int hipGraphExecDestroy(void *x) {
-  std::free(x);
+  delete static_cast<Graph *>(x);
   return 0;
 }
-int hipGraphLaunch(void *, void *) { return called("hipGraphLaunch"); }
+int hipGraphLaunch(void *x, void *) {
+  if (const int e = called("hipGraphLaunch")) return e;
+  std::lock_guard<std::mutex> lock(mu);
+  graph_nodes = static_cast<Graph *>(x)->nodes;
+  for (const Plan &q : static_cast<Graph *>(x)->plans) run_plan(q);
+  return 0;
+}
 
 }  // extern "C"

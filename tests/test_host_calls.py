@@ -17,7 +17,7 @@ PREAMBLE = """
 import ctypes, sys
 import numpy as np
 hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-for fn in ("calls", "launches", "live"):
+for fn in ("calls", "launches", "live", "flags_up", "graph_nodes"):
     getattr(hip, "fake_hip_" + fn).restype = ctypes.c_int64
 sys.path.insert(0, sys.argv[2])
 import dlbc_amd as D
@@ -156,4 +156,42 @@ def test_memory_is_made_on_the_device_of_its_lattice(run, current):
     import gc
     gc.collect()
     assert live(0) == 0 and live(1) == 0
+    """)
+
+
+FAILURES = [("hipLaunchKernel", 1), ("hipLaunchKernel", 2), ("hipStreamEndCapture", 1),
+            ("hipGraphInstantiate", 1), ("hipGraphLaunch", 1), ("hipGraphLaunch", 2),
+            ("hipGetLastError", 1), ("hipGetLastError", 2)]
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("what", ["lattice", "batch"])
+def test_flags_are_down_after_a_call_that_failed(run, what, graph):
+    """Every launch of the one-launch step starts with its flags down, also after
+    a call that failed before, within or after a capture, and no graph that is
+    short of a launch is kept."""
+    run(f"""
+    for name, nth in {FAILURES}:
+        for before in (0, 1, 32, 33):
+            if "{what}" == "lattice":
+                it = lattice((70, 80, 64))
+            else:
+                it = D.Batch([lattice((128, 128, 96), storage="f32_shift")])
+                it.set_config(8, 64, 512, 2)
+                if before == 33:
+                    it.autotune()
+                    it.set_config(8, 64, 512, 2)
+            it.step(before, graph={graph})
+            it.synchronize()
+            fail(name, nth)
+            try:
+                it.step(65, graph={graph})
+            except D.DlbcError:
+                pass
+            fail(name, 1 << 30)  # not planned any longer
+            for k in (1, 64, 33, 2, 65):
+                it.step(k, graph={graph})
+                if {graph} and k > 1:
+                    assert hip.fake_hip_graph_nodes() == (32 if "{what}" == "lattice" else 2)
+            assert hip.fake_hip_flags_up() == 0, (name, nth, before)
     """)
