@@ -815,6 +815,9 @@ int steps_per_launch(const dlbc_gpu_ctx *c) {
   return 1;
 }
 
+// The timer's slot of such a launch; its single steps take slot 0.
+constexpr int kStepsSlot = 1;
+
 // nsteps steps: launches on the library stream and swaps of the two population
 // buffers, nothing else (so they can be captured).
 int advance(dlbc_gpu_ctx *c, int sched, int nsteps, Timer *tm) {
@@ -823,10 +826,13 @@ int advance(dlbc_gpu_ctx *c, int sched, int nsteps, Timer *tm) {
   for (; per > 1 && t + per <= nsteps; t += per) {
     const double *A = static_cast<const double *>(c->popA);
     double *B = static_cast<double *>(c->popB);
+    tm->slot = kStepsSlot;
+    tm->before();
     if (per == multi_steps<8>())
       launch_single_multi<8>(A, B, c->nbw, c->geo, c->p, c->stream);
     else
       launch_single_multi<16>(A, B, c->nbw, c->geo, c->p, c->stream);
+    tm->after();
     std::swap(c->popA, c->popB);
   }
   for (; t < nsteps; ++t) {
@@ -1680,22 +1686,27 @@ int dlbc_gpu_step_timed(dlbc_gpu_ctx *c, int nsteps, double *elapsed_ms, double 
                         int *nkernels) {
   if (!c || nsteps < 1) return DLBC_ERR_ARG;
   int rc = prepare(c);
+  if (!rc) rc = split_ready(c);
   if (rc) return rc;
   double acc[kMaxKernels] = {0};
-  int nk = 0;
+  int launches[kMaxKernels] = {0}, nk = 0;
+  const int per = steps_per_launch(c);
   hipEvent_t t0 = c->ev[2 * kMaxKernels], t1 = c->ev[2 * kMaxKernels + 1];
   HIPCHK(c, hipEventRecord(t0, c->stream));
-  for (int t = 0; t < nsteps; ++t) {
+  for (int t = 0; t < nsteps;) {
+    const int n = nsteps - t >= per ? per : 1;  // the steps of a launch, as in advance()
     Timer tm{c, true};
-    rc = do_steps(c, 1, &tm);
+    rc = do_steps(c, n, &tm);
     if (rc) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    nk = tm.slot;
-    for (int k = 0; k < nk; ++k) {
+    for (int k = n > 1 ? kStepsSlot : 0; k < tm.slot; ++k) {
       float ms = 0;
       HIPCHK(c, hipEventElapsedTime(&ms, c->ev[2 * k], c->ev[2 * k + 1]));
       acc[k] += ms;
+      ++launches[k];
     }
+    nk = std::max(nk, tm.slot);
+    t += n;
   }
   HIPCHK(c, hipEventRecord(t1, c->stream));
   HIPCHK(c, hipEventSynchronize(t1));
@@ -1703,7 +1714,7 @@ int dlbc_gpu_step_timed(dlbc_gpu_ctx *c, int nsteps, double *elapsed_ms, double 
   HIPCHK(c, hipEventElapsedTime(&tot, t0, t1));
   if (elapsed_ms) *elapsed_ms = tot;
   if (kernel_ms)
-    for (int k = 0; k < nk; ++k) kernel_ms[k] = acc[k] / nsteps;
+    for (int k = 0; k < nk; ++k) kernel_ms[k] = launches[k] ? acc[k] / launches[k] : 0.0;
   if (nkernels) *nkernels = nk;
   return DLBC_OK;
 }
@@ -1712,6 +1723,7 @@ const char *dlbc_gpu_kernel_name(const dlbc_gpu_ctx *c, int i) {
   if (!c) return "";
   const int sched = effective_schedule(c);
   if (tile_step(c)) return i == 0 ? "tile_step" : "";
+  if (i == kStepsSlot && steps_per_launch(c) > 1) return "stream_collide_steps";
   if (sched == DLBC_SCHED_FUSED && c->storage != DLBC_STORAGE_F64)
     return i == 0 ? "tiled_d3q19_shifted" : "";
   if (sched == DLBC_SCHED_FUSED) return i == 0 ? "fused_d3q19" : "";

@@ -141,8 +141,11 @@ int dlbc_gpu_advect(dlbc_gpu_ctx *ctx);
 
 /* As dlbc_gpu_step, and report the elapsed GPU time of the nsteps (HIP
  * events on the library stream) and, per kernel of the schedule, the average
- * duration of one launch (kernel_ms[i], i < *nkernels, at most 8 entries;
- * events bracket every launch, so this mode adds a little overhead). */
+ * duration of one launch (kernel_ms[i], i < *nkernels, at most 8 entries, 0
+ * for a kernel that these steps did not launch; events bracket every launch
+ * and the host waits for each step, so this mode adds a little overhead).  On
+ * small single-component D2Q9 lattices kernel 1 is the launch of four or eight
+ * steps and kernel 0 the single step. */
 int dlbc_gpu_step_timed(dlbc_gpu_ctx *ctx, int nsteps, double *elapsed_ms, double *kernel_ms,
                         int *nkernels);
 /* Name of kernel slot i of the current schedule (static string). */

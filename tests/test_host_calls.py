@@ -195,3 +195,43 @@ def test_flags_are_down_after_a_call_that_failed(run, what, graph):
                     assert hip.fake_hip_graph_nodes() == (32 if "{what}" == "lattice" else 2)
             assert hip.fake_hip_flags_up() == 0, (name, nth, before)
     """)
+
+
+@pytest.mark.parametrize("n,nc,sc,steps,per", [((64, 64), 1, False, 35, 8), ((200, 200), 1, False, 6, 4),
+                                               ((64, 64), 1, False, 3, 8), ((64, 64), 1, False, 16, 8),
+                                               ((64, 64), 2, True, 5, 1), ((600, 600), 1, False, 5, 1),
+                                               ((20, 20, 20), 2, True, 3, 1)], ids=str)
+def test_timed_steps_launch_what_steps_launch(run, n, nc, sc, steps, per):
+    run(f"""
+    lat = lattice({n}, {nc}, {sc})
+    counts = []
+    for work in (lat.step, lat.step_timed):
+        before = [launches(k) for k in ("", "k_single_multi")]
+        out = work({steps})
+        counts.append([launches(k) - b for k, b in zip(("", "k_single_multi"), before)])
+    assert counts[0] == counts[1], counts
+    assert counts[0][1] == ({steps} // {per} if {per} > 1 else 0)
+    kernels = out[1]
+    if {per} > 1:  # a launch takes 1 ms on the stand-in
+        want = {{"stream_collide": 1.0 if {steps} % {per} else 0.0}}
+        if {steps} >= {per}:
+            want["stream_collide_steps"] = 1.0
+        assert kernels == want, kernels
+    else:
+        assert set(kernels.values()) == {{1.0}} and "" not in kernels
+    """)
+
+
+@pytest.mark.parametrize("storage,n", [("f64", (70, 80, 64)), ("f32_shift", (128, 128, 96))])
+def test_timed_steps_start_with_the_tables_made(run, storage, n):
+    run(f"""
+    lat = lattice({n}, storage="{storage}")
+    before = live(0)
+    fail("hipEventRecord", 1)  # the one that starts the time
+    try:
+        lat.step_timed(1)
+        assert False
+    except D.DlbcError:
+        pass
+    assert live(0) == before + 2
+    """)
