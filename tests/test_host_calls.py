@@ -235,3 +235,18 @@ def test_timed_steps_start_with_the_tables_made(run, storage, n):
         pass
     assert live(0) == before + 2
     """)
+
+
+@pytest.mark.parametrize("storage", ["f32_shift", "f16_shift"])
+def test_the_large_batch_takes_one_launch_per_step(run, storage):
+    from test_split_one_launch import BATCH
+    run(f"""
+    batch = D.Batch([lattice(n, storage="{storage}") for n in {BATCH}])
+    batch.set_config(8, 64, 512, 2)
+    batch.step(5, graph=False)
+    assert launches("batch_split_collide") == 5 and launches("batch_split_psi") == 0
+    batch = D.Batch(batch.members[:3])  # 5,907 blocks
+    batch.set_config(8, 64, 512, 2)
+    batch.step(5, graph=False)
+    assert launches("batch_split_collide") == 10 and launches("batch_split_psi") == 5
+    """)

@@ -126,3 +126,50 @@ def test_thin_planes_and_long_rows_equal_oracle(D, n, kernels):
     g.step(1)
     o.run(3)
     _same(g, o, n)
+
+
+# 6,187 blocks of 256 sites: past the 6,000 from which a batch takes one launch
+# (that it does is counted in test_host_calls.py), with a member of one block
+BATCH = [(70, 83, 91), (4, 4, 4), (64, 96, 160), (33, 70, 31)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage,solid", [("f32_shift", False), ("f32_shift", True),
+                                           ("f16_shift", False)])
+def test_large_batch_equals_lattices_alone(D, storage, solid):
+    """One launch per step over all members: eager, graph and odd step counts, a
+    member whose Shan-Chen force goes off and on in between, one with
+    self-coupling, and one of other solids than its neighbours."""
+    ps = [_params(n, ("BDist2", "SecondOrder")[k % 2], solid and k != 3)
+          for k, n in enumerate(BATCH)]
+    ps[0]["gcc"] = [[0.4, 3.0], [3.0, -0.3]]
+    alone, members = ([D.Lattice.from_params(p, storage=storage) for p in ps] for _ in range(2))
+    for lat in alone:
+        lat.set_block_order(8)  # two launches
+    batch = D.Batch(members)
+    batch.set_config(8, 64, 512, 2)
+    for k, graph, on in ((4, True, True), (3, False, True), (2, True, False), (1, False, False),
+                         (7, True, True), (5, True, True), (1, True, True)):
+        for lats in (alone, members):
+            p = ps[2]
+            lats[2].set_params(p["tau"], p["gcc"], p.get("gwc"), None, None, p["eqDistForm"],
+                               "Exponential", on)
+        batch.step(k, graph=graph)
+        for lat in alone:
+            lat.step(k)
+        batch.synchronize()
+        for a, b, n in zip(alone, members, BATCH):
+            _same(a, b, (n, k))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [(70, 90, 61), (16, 200, 128)], ids=str)
+@pytest.mark.parametrize("solid", [True, False])
+def test_f64_self_coupling_equals_oracle(D, n, solid):
+    from oracle.oracle import Oracle
+    p = dict(_params(n, "BDist2", solid), gcc=[[0.4, 3.0], [3.0, -0.3]])
+    g, o = D.Lattice.from_params(p, schedule="split"), Oracle.from_params(p)
+    assert list(g.step_timed(1)[1]) == ["split_one_launch"]
+    g.step(2)
+    o.run(3)
+    _same(g, o, n)
