@@ -1001,7 +1001,7 @@ int field_to_host(dlbc_gpu_ctx *c, int kind, int f1, int f2, int k, double *host
         host_pieces(c, halo, site_bytes, host, 0, bytes, [&](char *to, size_t at, size_t len) {
           std::memcpy(to, static_cast<const char *>(s.p) + at, len);
         });
-      slot_pool().give(s);
+      if (e == hipSuccess) slot_pool().give(s);  // (else the kernel may still write to it)
       return rc;
     }
   }

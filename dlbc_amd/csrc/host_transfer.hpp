@@ -114,19 +114,24 @@ inline SlotPool &slot_pool() {
   return *pool;
 }
 
-// work(slot, k) for the parts k = 0 .. parts-1 of a transfer, each thread with a
-// slot of its own.  Returns the first error; without a pinned slot
+// work(slot, k) for the parts k = 0 .. parts-1 of a transfer on `stream`, each
+// thread with a slot of its own.  Returns the first error; without a pinned slot
 // hipErrorOutOfMemory before any part is done.
 template <class Work>
-inline hipError_t transfer_parts(int device, int parts, Work work) {
+inline hipError_t transfer_parts(int device, hipStream_t stream, int parts, Work work) {
   PinnedSlot mine = slot_pool().take(device);
   if (!mine.p) return hipErrorOutOfMemory;
   std::atomic<int> next{0};
   std::atomic<int> err{(int)hipSuccess};
-  auto run = [&](const PinnedSlot &s) {
+  auto run = [&](PinnedSlot &s) {
     for (int k; err.load() == hipSuccess && (k = next.fetch_add(1)) < parts;) {
       const hipError_t e = work(s, k);
-      if (e != hipSuccess) err.store((int)e);
+      if (e == hipSuccess) continue;
+      err.store((int)e);
+      // a copy may be under way in the slot: where that cannot be waited for, the
+      // slot is left alone for good
+      if (hipStreamSynchronize(stream) != hipSuccess) s = PinnedSlot{};
+      return;
     }
   };
   std::vector<std::thread> threads;
@@ -153,7 +158,7 @@ template <class Put>
 inline hipError_t transfer_down(int device, hipStream_t stream, const void *dev, size_t bytes,
                                 Put put) {
   const int parts = (int)((bytes + kSlotBytes - 1) / kSlotBytes);
-  return transfer_parts(device, parts, [&](const PinnedSlot &s, int k) {
+  return transfer_parts(device, stream, parts, [&](const PinnedSlot &s, int k) {
     const size_t o = (size_t)k * kSlotBytes, n = std::min(kSlotBytes, bytes - o);
     hipError_t e = hipMemcpyAsync(s.p, static_cast<const char *>(dev) + o, n,
                                   hipMemcpyDeviceToHost, stream);
@@ -169,7 +174,7 @@ inline hipError_t transfer_down(int device, hipStream_t stream, const void *dev,
 template <class Get>
 inline hipError_t transfer_up(int device, hipStream_t stream, void *dev, size_t bytes, Get get) {
   const int parts = (int)((bytes + kSlotBytes - 1) / kSlotBytes);
-  return transfer_parts(device, parts, [&](const PinnedSlot &s, int k) {
+  return transfer_parts(device, stream, parts, [&](const PinnedSlot &s, int k) {
     const size_t o = (size_t)k * kSlotBytes, n = std::min(kSlotBytes, bytes - o);
     get(o, static_cast<char *>(s.p), n);
     hipError_t e = hipMemcpyAsync(static_cast<char *>(dev) + o, s.p, n, hipMemcpyHostToDevice,

@@ -11,6 +11,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -19,7 +20,7 @@ namespace {
 std::mutex mu;
 std::map<std::string, int64_t> calls, launches;
 struct Failure {
-  int64_t in;  // calls until it
+  int64_t in;  // calls until it; 0: every call
   int code;
 };
 std::map<std::string, Failure> failures;
@@ -34,10 +35,14 @@ int called(const char *name) {
   std::lock_guard<std::mutex> lock(mu);
   ++calls[name];
   auto f = failures.find(name);
-  if (f == failures.end() || --f->second.in > 0) return 0;
-  const int code = f->second.code;
-  failures.erase(f);
-  return last_error = code;
+  if (f == failures.end()) return 0;
+  const Failure now = f->second;
+  if (now.in > 1) {
+    --f->second.in;
+    return 0;
+  }
+  if (now.in == 1) failures.erase(f);
+  return last_error = now.code;
 }
 
 void *made(void *p) {
@@ -90,6 +95,24 @@ struct Graph {
 std::map<void *, Graph> capturing;  // by stream
 int64_t graph_nodes = 0;            // kernels of the graph launched last
 
+// Pinned memory that copies queued on a stream still use: until the stream, or an
+// event recorded after them by their thread, was waited for.
+std::set<const void *> pinned;
+std::map<const void *, void *> busy;  // pinned memory -> stream
+std::map<const void *, const void *> recorded_after;  // event -> pinned memory
+thread_local const void *last_used = nullptr;
+int64_t busy_used = 0;
+void uses(const void *p, void *stream) {
+  if (!pinned.count(p)) return;
+  if (busy.count(p)) ++busy_used;
+  busy[p] = stream;
+  last_used = p;
+}
+void waited(void *stream) {
+  for (auto it = busy.begin(); it != busy.end();)
+    it = it->second == stream ? busy.erase(it) : std::next(it);
+}
+
 struct Dim3 {
   uint32_t x, y, z;
 };
@@ -131,7 +154,12 @@ int64_t fake_hip_graph_nodes() {
   std::lock_guard<std::mutex> lock(mu);
   return graph_nodes;
 }
-// The nth call of `name` from now on returns `code`.
+// Pinned memory used again or freed while a copy may be under way in it.
+int64_t fake_hip_busy_used() {
+  std::lock_guard<std::mutex> lock(mu);
+  return busy_used;
+}
+// The nth call of `name` from now on returns `code`, or every call (nth 0).
 void fake_hip_fail(const char *name, int nth, int code) {
   std::lock_guard<std::mutex> lock(mu);
   failures[name] = {nth, code};
@@ -220,10 +248,17 @@ int hipHostMalloc(void **p, size_t n, unsigned) {
   *p = nullptr;
   if (const int e = called("hipHostMalloc")) return e;
   *p = made(std::calloc(n, 1));
+  std::lock_guard<std::mutex> lock(mu);
+  pinned.insert(*p);
   return 0;
 }
 int hipHostFree(void *p) {
   if (const int e = called("hipHostFree")) return e;
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (busy.count(p)) ++busy_used;
+    pinned.erase(p);
+  }
   return gone(p);
 }
 int hipGetSymbolAddress(void **p, const void *) {
@@ -236,9 +271,12 @@ int hipMemcpy(void *to, const void *from, size_t n, int) {
   std::memcpy(to, from, n);
   return 0;
 }
-int hipMemcpyAsync(void *to, const void *from, size_t n, int, void *) {
+int hipMemcpyAsync(void *to, const void *from, size_t n, int, void *stream) {
   if (const int e = called("hipMemcpyAsync")) return e;
   std::memcpy(to, from, n);
+  std::lock_guard<std::mutex> lock(mu);
+  uses(to, stream);
+  uses(from, stream);
   return 0;
 }
 int hipMemsetAsync(void *p, int v, size_t n, void *) {
@@ -254,7 +292,12 @@ int hipStreamDestroy(void *s) {
   std::free(s);
   return 0;
 }
-int hipStreamSynchronize(void *) { return called("hipStreamSynchronize"); }
+int hipStreamSynchronize(void *stream) {
+  if (const int e = called("hipStreamSynchronize")) return e;
+  std::lock_guard<std::mutex> lock(mu);
+  waited(stream);
+  return 0;
+}
 int hipStreamWaitEvent(void *, void *, unsigned) { return 0; }
 int hipEventCreateWithFlags(void **e, unsigned) {
   *e = nullptr;
@@ -264,8 +307,18 @@ int hipEventCreateWithFlags(void **e, unsigned) {
 }
 int hipEventCreate(void **e) { return hipEventCreateWithFlags(e, 0); }
 int hipEventDestroy(void *e) { return gone(e); }
-int hipEventRecord(void *, void *) { return called("hipEventRecord"); }
-int hipEventSynchronize(void *) { return called("hipEventSynchronize"); }
+int hipEventRecord(void *event, void *) {
+  if (const int e = called("hipEventRecord")) return e;
+  std::lock_guard<std::mutex> lock(mu);
+  recorded_after[event] = last_used;
+  return 0;
+}
+int hipEventSynchronize(void *event) {
+  if (const int e = called("hipEventSynchronize")) return e;
+  std::lock_guard<std::mutex> lock(mu);
+  busy.erase(recorded_after[event]);
+  return 0;
+}
 int hipEventElapsedTime(float *ms, void *, void *) {
   *ms = 1.0f;
   return 0;

@@ -17,7 +17,7 @@ PREAMBLE = """
 import ctypes, sys
 import numpy as np
 hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-for fn in ("calls", "launches", "live", "flags_up", "graph_nodes"):
+for fn in ("calls", "launches", "live", "flags_up", "graph_nodes", "busy_used"):
     getattr(hip, "fake_hip_" + fn).restype = ctypes.c_int64
 sys.path.insert(0, sys.argv[2])
 import dlbc_amd as D
@@ -249,4 +249,31 @@ def test_the_large_batch_takes_one_launch_per_step(run, storage):
     batch.set_config(8, 64, 512, 2)
     batch.step(5, graph=False)
     assert launches("batch_split_collide") == 10 and launches("batch_split_psi") == 5
+    """)
+
+
+@pytest.mark.parametrize("n", [(16, 16, 16), (40, 40, 40)], ids=str)
+@pytest.mark.parametrize("name", ["hipMemcpyAsync", "hipEventRecord", "hipEventSynchronize"])
+@pytest.mark.parametrize("stuck", [False, True])
+def test_pinned_memory_is_not_used_again_while_a_copy_may_be_under_way(run, n, name, stuck):
+    """After a transfer that failed between its copy and the wait for it, also
+    where the stream cannot be waited for."""
+    run(f"""
+    pop = np.random.default_rng(1).random({n} + (19,))
+    for nth in (1, 2, 3):
+        a, b = lattice({n}), lattice({n})
+        for work in (lambda: a.upload_population(0, pop), lambda: a.population(0)):
+            fail("{name}", nth)
+            if {stuck}:
+                fail("hipStreamSynchronize", 0)
+            try:
+                work()
+            except D.DlbcError:
+                pass
+            fail("{name}", 1 << 30)
+            fail("hipStreamSynchronize", 1 << 30)
+            b.upload_population(0, pop)
+            b.population(0)
+        del a, b
+    assert hip.fake_hip_busy_used() == 0, hip.fake_hip_busy_used()
     """)
