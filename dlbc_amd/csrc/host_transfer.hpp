@@ -60,6 +60,7 @@ struct SlotPool {
   std::vector<PinnedSlot> idle;
   int users = 0;
 
+  SlotPool() { idle.reserve(kTransferKept); }  // (give() is called from threads and never throws)
   static void drop(PinnedSlot s) {
     if (s.done) (void)hipEventDestroy(s.done);
     if (s.p) (void)hipHostFree(s.p);
