@@ -601,18 +601,25 @@ bool split_one_launch(const dlbc_gpu_ctx *c) {
 }
 
 // Whether a step is one launch over small tiles (kernels_tile.hpp): D2Q9 with
-// Shan-Chen under the automatic schedule.  With one or two components in the
-// middle range, where both buffers stay in the memory-side cache and the
-// arithmetic of the border decides, two launches are faster (us per step, two
-// launches / one, two components: 400^2 18.9 / 17.1, 450^2 21.4 / 23.3, 850^2
-// 59 / 71, 1024^2 84 / 85, 1400^2 173 / 165, 2048^2 351 / 323); three and more
-// gain everywhere (300^2 21 / 19, 1024^2 154 / 149).  The kernel's 32-bit
-// offsets within a component need 9 sp 8 < 2^32.
+// Shan-Chen under the automatic schedule.  On large lattices the launches'
+// latency no longer counts and the border's arithmetic does: with one or two
+// components from 160,000 sites on (us per step, two launches / one, two
+// components: 400^2 18.9 / 17.1, 450^2 21.4 / 23.3, 1024^2 84 / 85, 1500^2 201 /
+// 210, 3001^2 750 / 890), with three from 1.1 million on (1024^2 154 / 149,
+// 1225^2 221 / 239, 1800^2 451 / 475), with four nowhere (2000^2 851 / 725).  And
+// tiles that stand over the end of an axis are computed whole: beyond 1,024 of
+// them, about one round of workgroups, four fifths of their cells have to be
+// sites (three components, 24000 x 2 15 / 38, x 4 19 / 37, x 9 33 / 41, x 12 42 /
+// 43; 4096 x 2, 1024 tiles, 13.6 / 11.4).  The kernel's 32-bit offsets within a
+// component need 9 sp 8 < 2^32.
 bool tile_step(const dlbc_gpu_ctx *c) {
   if (c->schedule != DLBC_SCHED_AUTO || c->storage != DLBC_STORAGE_F64 || !c->p.sc || c->d != 2)
     return false;
   if (9 * 8 * c->geo.sp >= (int64_t)1 << 32) return false;
-  return c->C > 2 || c->geo.sites <= 160000 || c->geo.sites >= 1500000;
+  const int64_t tiles =
+      (int64_t)blocks_for(c->geo.nx, kTileX) * blocks_for(c->geo.ny, kTileY);
+  if (tiles > 1024 && 5 * (int64_t)c->geo.sites < 4 * kTileSites * tiles) return false;
+  return c->geo.sites <= (c->C <= 2 ? 160000 : (c->C == 3 ? 1100000 : INT32_MAX));
 }
 
 // While a call launches steps, and until it has done so without an error, the

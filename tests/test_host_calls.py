@@ -277,3 +277,20 @@ def test_pinned_memory_is_not_used_again_while_a_copy_may_be_under_way(run, n, n
         del a, b
     assert hip.fake_hip_busy_used() == 0, hip.fake_hip_busy_used()
     """)
+
+
+@pytest.mark.parametrize("n,nc,tile", [
+    ((64, 64), 2, True), ((400, 400), 2, True), ((2048, 2048), 2, False), ((3001, 3001), 1, False),
+    ((1024, 1024), 3, True), ((1225, 1225), 3, False), ((1225, 1225), 4, True),
+    ((50000, 2), 2, False), ((24000, 4), 3, False), ((3, 500000), 4, False), ((4096, 2), 2, True),
+    ((2, 8192), 1, True), ((24000, 16), 4, True), ((24000, 13), 4, True), ((24000, 12), 4, False)],
+    ids=str)
+def test_tiles_of_a_d2q9_step_are_mostly_sites(run, n, nc, tile):
+    """Thin lattices, of whose tiles most cells are no sites, and large ones take
+    two launches per step."""
+    run(f"""
+    lat = lattice({n}, {nc})
+    lat.step(3)
+    assert launches("k_tile_step") == {3 if tile else 0}
+    assert launches("5k_psi") == {0 if tile else 3}
+    """)
