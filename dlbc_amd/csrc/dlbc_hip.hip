@@ -811,14 +811,17 @@ int step_once(dlbc_gpu_ctx *c, int sched, Timer *tm) {
 // still beats single steps.  us per step, single (eager / graph), four, eight:
 // 64^2 4.3 / 2.9, 2.4, 1.85; 128^2 4.5 / 3.4, 2.6, 2.0; 192^2 4.9 / 4.1, 3.1, 5.0;
 // 256^2 5.7 / 5.0, 3.4, 6.6; 300^2 6.5 / 6.1, 5.2; 400^2 8.7 / 8.5, 7.0; 512^2 8.3,
-// 9.3.
+// 9.3.  Beyond one round three fifths of the tiles' cells have to be sites: 4706 x
+// 17 (0.53 of them) 5.6, 6.1; 4000 x 20 (0.62) 5.5, 4.7.
 int steps_per_launch(const dlbc_gpu_ctx *c) {
   if (c->schedule != DLBC_SCHED_AUTO || c->storage != DLBC_STORAGE_F64 || c->d != 2 ||
       c->C != 1 || c->p.sc)
     return 1;
   auto tiles = [&](int t) { return (int64_t)((c->n[0] + t - 1) / t) * ((c->n[1] + t - 1) / t); };
   if (tiles(8) <= 256) return multi_steps<8>();
-  if (tiles(16) <= 256 || (tiles(16) <= 650 && c->geo.sites >= 80000)) return multi_steps<16>();
+  if (tiles(16) <= 256 || (tiles(16) <= 650 && c->geo.sites >= 80000 &&
+                           5 * (int64_t)c->geo.sites >= 3 * 256 * tiles(16)))
+    return multi_steps<16>();
   return 1;
 }
 

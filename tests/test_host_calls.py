@@ -294,3 +294,15 @@ def test_tiles_of_a_d2q9_step_are_mostly_sites(run, n, nc, tile):
     assert launches("k_tile_step") == {3 if tile else 0}
     assert launches("5k_psi") == {0 if tile else 3}
     """)
+
+
+@pytest.mark.parametrize("n,per", [((64, 64), 8), ((2000, 2), 8), ((256, 256), 4), ((2000, 17), 4),
+                                   ((400, 400), 4), ((4000, 20), 4), ((4706, 17), 1),
+                                   ((17, 4706), 1), ((500, 500), 1)], ids=str)
+def test_steps_of_a_launch(run, n, per):
+    """More than one round of workgroups only where their tiles are mostly sites."""
+    run(f"""
+    lat = lattice({n}, 1, False)
+    lat.step(8)
+    assert launches("k_single") == 8 // {per}, launches("k_single")
+    """)
