@@ -21,10 +21,11 @@ namespace dlbc {
 // Threads of a workgroup: one wave, so that small lattices reach every CU.
 constexpr int kSingleThreads = 64;
 
-// Nontemporal stores where the two buffers exceed the memory-side cache: 256^3 906
-// without and 873 us with, 160^3 with plates 219 and 211; 70x45x98, which stays
-// in it, 18.8 and 21.0.
-constexpr int64_t kSingleCached = 256ll << 20;
+// Nontemporal stores where the two buffers exceed the memory-side cache by some
+// (us per step, without / with): D3Q19 96^3 (257 MiB) 45.1 / 47.6, 100^3 (290 MiB)
+// 53.9 / 53.8, 112^3 78 / 74, 256^3 906 / 873; D2Q9 1300^2 (232 MiB) 40.6 / 42.5,
+// 1400^2 (269 MiB) 49.2 / 49.0, 1600^2 66 / 63; 70x45x98 18.8 / 21.0.
+constexpr int64_t kSingleCached = 288ll << 20;
 
 // Whether the kernel serves a lattice: neighbours one site away on every axis
 // (not D1Q5), and 32-bit byte offsets.

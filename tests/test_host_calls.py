@@ -306,3 +306,20 @@ def test_steps_of_a_launch(run, n, per):
     lat.step(8)
     assert launches("k_single") == 8 // {per}, launches("k_single")
     """)
+
+
+@pytest.mark.parametrize("n,nt", [((96, 96, 96), 0), ((99, 99, 99), 0), ((100, 100, 100), 1),
+                                  ((1400, 1400), 0), ((1500, 1500), 1)], ids=str)
+@pytest.mark.parametrize("solid", [0, 1])
+def test_single_component_stores_past_the_cache(run, n, nt, solid):
+    """Nontemporal stores (the kernel's last template argument) from where both
+    buffers no longer stay in the memory-side cache."""
+    run(f"""
+    lat = lattice({n}, 1, False)
+    if {solid}:
+        mask = np.zeros({n}, np.int32)
+        mask[0] = 1
+        lat.upload_mask(mask)
+    lat.step(2)
+    assert launches("k_singleI") == launches("Lb{solid}ELb{nt}EEEvPK") == 2
+    """)
