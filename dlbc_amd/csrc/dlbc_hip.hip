@@ -584,20 +584,39 @@ int order_strip(int storage) {
   return storage == DLBC_STORAGE_F16_SHIFT ? kOrderStripF16 : kOrderStrip;
 }
 
+// Blocks of a row in the one-launch order at most.
+int order_row_most(int storage) {
+  return storage == DLBC_STORAGE_F16_SHIFT ? kOrderRowMostF16 : kOrderRowMost;
+}
+
 // Whether a Shan-Chen step of the split schedule is one launch.  us per step,
 // two launches against one: FP64 48^3 22 / 34, 64^3 42.6 / 42.5, 72^3 63.5 /
 // 61.3, 96^3 148 / 135, 256^3 2960 / 2254; FP32 80^3 42 / 48, 96^3 70 / 73,
 // 190x151x117 with solids 292 / 249, 256^3 1390 / 1120; FP16 without solids
 // 128^3 91 / 90, 256^3 719 / 657, 384^3 2570 / 2310.  FP16 with solids, whose
 // collide is bound by its instructions and whose psi then runs at the collide's
-// four waves per SIMD, 836 / 943 at 256^3: two launches.  Lattices of thin planes
-// or very long rows keep two launches, too (split_order_serves).
+// four waves per SIMD, 836 / 943 at 256^3: two launches.
+// Where a collide waits for more than its neighbourhood, a lattice has to be
+// larger: rows of 32 blocks and more (FP64 10 x 11 x 4096 72 / 77, 16 x 17 x 4096
+// 185 / 169, 5 x 5 x 16384 67 / 73, 8 x 8 x 16384 176 / 171; FP32 7 x 9 x 24569 121
+// / 131, 9 x 10 x 24569 187 / 179; FP16 16 x 17 x 8192 98 / 100, 25 x 26 x 8192 236
+// / 229) and, in FP16, planes of one block (6100 x 16 x 16 67 / 76, 40000 x 16 x
+// 16 489 / 456).  Thinner planes and longer rows keep two launches
+// (split_order_serves).
 bool split_one_launch(const dlbc_gpu_ctx *c) {
   if (c->d != 3 || c->C != 2 || !c->p.sc || c->geo.order_chunk != 0 || c->one_launch_off)
     return false;
-  if (c->storage == DLBC_STORAGE_F16_SHIFT && c->has_solid) return false;
-  const int64_t blocks = c->storage == DLBC_STORAGE_F64 ? 2500 : 6000;
-  return c->geo.sites >= blocks * split_sites(c) && split_order_serves(c->geo, split_sites(c));
+  const bool f16 = c->storage == DLBC_STORAGE_F16_SHIFT;
+  if (f16 && c->has_solid) return false;
+  const int sb = split_sites(c);
+  const bool long_rows = c->geo.nz >= 32 * sb;
+  int least = c->storage == DLBC_STORAGE_F64 ? 2500 : 6000;
+  if (f16 && (long_rows || (int64_t)c->geo.ny * c->geo.nz < 2 * sb))
+    least = 20000;
+  else if (long_rows)
+    least = 8000;
+  return c->geo.sites >= (int64_t)least * sb &&
+         split_order_serves(c->geo, sb, order_row_most(c->storage));
 }
 
 // Whether a step is one launch over small tiles (kernels_tile.hpp): D2Q9 with
@@ -2124,7 +2143,7 @@ bool batch_one_launch(const dlbc_batch *b) {
   if (b->storage == DLBC_STORAGE_F16_SHIFT && batch_has_solid(b)) return false;
   if (b->h_first.back() < 6000) return false;
   for (auto *c : b->ctx)
-    if (!split_order_serves(c->geo, kShiftSites)) return false;
+    if (!split_order_serves(c->geo, kShiftSites, order_row_most(b->storage))) return false;
   return true;
 }
 

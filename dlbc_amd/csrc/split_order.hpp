@@ -104,18 +104,18 @@ __host__ __device__ inline void split_needs(const Geo &g, int SB, int blk, int k
 // Both are few where a block meets no more than two planes (planes of a block's
 // sites or more; a block over more planes would wait for the whole lattice) and
 // rows are not too long, of which a collide waits for nine whole ones.  us per
-// step, two launches / one: FP64 rows of 16, 128, 256 and 512 blocks (16 x 16
-// rows) 361 / 314, 715 / 656, 1442 / 1441 and 2936 / 3128; FP32 rows of 128, 256
-// and 512 blocks 715 / 636, 1426 / 1384 and 366 / 390; planes of one block
-// (16384 x 8 x 16) FP64 347 / 290, FP32 (8192 x 16 x 16) 173 / 153.  A lattice of
-// no more than kOrderRowBlocks blocks (a member of a batch) has no more to wait
-// for than such a row.  (Components of whole tiles of 64 sites: no line of psi
-// holds sites of two waves.)
-constexpr int kOrderRowBlocks = 256;
-inline bool split_order_serves(const Geo &g, int SB) {
-  const int64_t most = (int64_t)kOrderRowBlocks * SB;
+// step of large lattices, two launches / one: FP64 rows of 16, 64, 128, 192 and
+// 512 blocks 316 / 279, 311 / 277, 304 / 292, 308 / 320 and 2936 / 3128; FP32 rows
+// of 64, 128, 192 and 512 blocks 756 / 644, 749 / 666, 768 / 751 and 366 / 390, and
+// of 192 in a smaller lattice 175 / 192; FP16 rows of 64 and 128 blocks 400 / 393
+// and 399 / 409.  A lattice of no more than kOrderAll blocks (a member of a batch)
+// has no more to wait for than such rows.  (Components of whole tiles of 64 sites:
+// no line of psi holds sites of two waves.)
+constexpr int kOrderAll = 256, kOrderRowMost = 128, kOrderRowMostF16 = 64;
+inline bool split_order_serves(const Geo &g, int SB, int row_most = kOrderRowMost) {
   if (g.sp % 64 != 0) return false;
-  return g.sites <= most || ((int64_t)g.ny * g.nz >= SB && g.nz <= most);
+  return g.sites <= (int64_t)kOrderAll * SB ||
+         ((int64_t)g.ny * g.nz >= SB && g.nz <= (int64_t)row_most * SB);
 }
 
 // The psi blocks and the collide blocks of a lattice in the order of their

@@ -97,10 +97,16 @@ def test_a_batch_keeps_a_graph_of_each_flag_set(run, n, steps):
 
 @pytest.mark.parametrize("storage,n,one", [
     ("f64", (100000, 10, 10), False), ("f64", (20000, 4, 4), False), ("f64", (4, 4, 65536), False),
-    ("f64", (16384, 8, 16), True), ("f64", (2, 5, 32768), True), ("f64", (128, 4, 4096), True),
-    ("f32_shift", (7000, 15, 16), False), ("f32_shift", (5, 5, 65537), False),
-    ("f32_shift", (8192, 16, 16), True), ("f32_shift", (5, 5, 65536), True),
-    ("f16_shift", (100000, 10, 10), False), ("f16_shift", (8192, 16, 16), True)], ids=str)
+    ("f64", (2500, 8, 16), True), ("f64", (25, 25, 520), True), ("f64", (41, 3, 2620), True),
+    ("f64", (10, 11, 4096), False), ("f64", (15, 17, 4096), True), ("f64", (4, 4, 20000), False),
+    ("f64", (8, 8, 16384), True), ("f64", (16, 8, 16385), False),
+    ("f32_shift", (7000, 15, 16), False), ("f32_shift", (6100, 16, 16), True),
+    ("f32_shift", (7, 9, 24569), False), ("f32_shift", (9, 10, 24569), True),
+    ("f32_shift", (16, 16, 32768), True), ("f32_shift", (16, 16, 32769), False),
+    ("f16_shift", (100000, 10, 10), False), ("f16_shift", (12000, 16, 16), False),
+    ("f16_shift", (40000, 16, 16), True), ("f16_shift", (3200, 16, 32), True),
+    ("f16_shift", (20, 20, 8192), False), ("f16_shift", (25, 26, 8192), True),
+    ("f16_shift", (32, 32, 16384), True), ("f16_shift", (32, 32, 16385), False)], ids=str)
 def test_thin_planes_and_long_rows_take_two_launches(run, storage, n, one):
     """A block of sites that meets more than two planes would wait for the whole
     lattice, and long rows for many blocks."""
@@ -109,14 +115,21 @@ def test_thin_planes_and_long_rows_take_two_launches(run, storage, n, one):
     lat.step(3)
     assert launches("split_psi") == {0 if one else 3}, launches("split_psi")
     assert launches("split_collide") == 3
-    if "{storage}" != "f64":
-        # a large member of this shape decides for its batch, a small one does not
-        for other in ((128, 128, 96), (1000, 4, 4)):
-            batch = D.Batch([lattice(other, storage="{storage}"), lat])
-            batch.set_config(8, 64, 512, 2)
-            psi = launches("batch_split_psi")
-            batch.step(3)
-            assert launches("batch_split_psi") - psi == {0 if one else 3}
+    """)
+
+
+@pytest.mark.parametrize("n,one", [((1000, 4, 4), True), ((4096, 4, 4), True), ((4097, 4, 4), False),
+                                   ((4, 5, 32768), True), ((4, 5, 32769), False),
+                                   ((7, 9, 24569), True)], ids=str)
+def test_thin_planes_and_long_rows_of_a_batch_member(run, n, one):
+    """A large member of such a shape decides for its batch, a small one does not."""
+    run(f"""
+    batch = D.Batch([lattice((128, 128, 96), storage="f32_shift"),
+                     lattice({n}, storage="f32_shift")])
+    batch.set_config(8, 64, 512, 2)
+    batch.step(3, graph=False)
+    assert launches("batch_split_collide") == 3
+    assert launches("batch_split_psi") == {0 if one else 3}
     """)
 
 

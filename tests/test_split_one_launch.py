@@ -113,12 +113,12 @@ def test_batch_in_one_launch_equals_lattices_alone(D, storage, solid):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,kernels", [((21000, 4, 4), 2), ((5, 2, 32769), 2), ((2600, 8, 16), 1),
-                                       ((5, 2, 32768), 1)], ids=str)
+@pytest.mark.parametrize("n,kernels", [((21000, 4, 4), 2), ((5, 13, 16385), 2), ((2600, 8, 16), 1),
+                                       ((7, 9, 16384), 2), ((5, 13, 16384), 1)], ids=str)
 def test_thin_planes_and_long_rows_equal_oracle(D, n, kernels):
-    """Planes of fewer sites than a block and rows of more than 256 blocks take
-    two launches; planes of one block and rows of 256 are the smallest and the
-    longest that take one."""
+    """Planes of fewer sites than a block and rows of more than 128 blocks take
+    two launches; planes of one block and, in a large lattice, rows of 128 are
+    the smallest and the longest that take one."""
     from oracle.oracle import Oracle
     p = _params(n, "BDist2", False)
     g, o = D.Lattice.from_params(p, schedule="split"), Oracle.from_params(p)
