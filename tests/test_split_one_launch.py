@@ -114,7 +114,7 @@ def test_batch_in_one_launch_equals_lattices_alone(D, storage, solid):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,kernels", [((21000, 4, 4), 2), ((5, 13, 16385), 2), ((2600, 8, 16), 1),
-                                       ((7, 9, 16384), 2), ((5, 13, 16384), 1)], ids=str)
+                                       ((6, 9, 16384), 2), ((5, 13, 16384), 1)], ids=str)
 def test_thin_planes_and_long_rows_equal_oracle(D, n, kernels):
     """Planes of fewer sites than a block and rows of more than 128 blocks take
     two launches; planes of one block and, in a large lattice, rows of 128 are
