@@ -144,14 +144,18 @@ void apply_block_order(dlbc_gpu_ctx *c, int chunk) {
 // value (FP64 storage) or w_i rho0_f + the stored deviation (shifted storage).
 template <int Q>
 struct LoadF64 {
+  static constexpr bool walks = true;
   const double *A;
   int64_t sp;
+  // from the site's tile_elem
+  __device__ double at(int f, int i, int64_t e) const { return A[f * (Q * sp) + 64 * i + e]; }
   __device__ double operator()(int f, int i, int s) const {
     return A[pop_elem_f64<Q>(f, i, s, sp)];
   }
 };
 template <class St>
 struct LoadShift {
+  static constexpr bool walks = false;
   const St *A;
   int64_t sp;
   double rho0[4];
@@ -355,11 +359,19 @@ __global__ void __launch_bounds__(256) k_reduce1(Ld ld, const uint8_t *__restric
   const int begin = b * chunk;
   const int end = min(begin + chunk, g.sites);
   DD acc{0.0, 0.0};
-  for (int s = begin + t; s < end; s += 256) {
+  // a thread's sites are four tiles apart: in FP64 with solids 128^3 takes 406 us
+  // so and 434 with the place formed for each site; FP32 64^3 246 and 178
+  int64_t e = tile_elem<L::q>(begin + t);
+  for (int s = begin + t; s < end; s += 256, e += 256 * L::q) {
     if (has_solid && mask[s]) continue;
     double n[L::q];
 #pragma unroll
-    for (int i = 0; i < L::q; ++i) n[i] = ld(f, i, s);
+    for (int i = 0; i < L::q; ++i) {
+      if constexpr (Ld::walks)
+        n[i] = ld.at(f, i, e);
+      else
+        n[i] = ld(f, i, s);
+    }
     double v;
     if (what == 0) {
       v = density<L>(n);
