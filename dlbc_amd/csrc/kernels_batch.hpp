@@ -354,9 +354,12 @@ __device__ inline int batch_block_lattice(const int *__restrict__ first, int nla
   return lo;
 }
 
-// SOLID: some member has solid sites (one without has all-zero solid words and
-// takes the same arithmetic path).  Without, the collide takes 88 VGPRs instead
-// of 122: five waves per SIMD.
+// SOLID: some member has solid sites.  Without, the collide takes 88 VGPRs instead
+// of 122: five waves per SIMD.  In two launches a member without solids still takes
+// the blocks without, in a batch with one member of solids (us per step, as all
+// others / so: FP16 40 members of 32^3 to 96^3 637 / 617, 8 of 48^3 54.0 / 51.6,
+// FP32 8 of 48^3 81.2 / 79.1).  In one launch it has all-zero solid words and goes
+// the same way as the others.
 template <class Store, bool SOLID, bool OFF32>
 __global__ void __launch_bounds__(kShiftThreads)
     k_batch_split_psi(const BatchLattice *__restrict__ lats, const int *__restrict__ first,
@@ -368,8 +371,11 @@ __global__ void __launch_bounds__(kShiftThreads)
   const Geo g = B.g;
   const ShiftParams p = B.p;
   if (!p.sc) return;  // this member's collide pass reads no psi
-  ssplit_psi_block<Store, SOLID, OFF32>(static_cast<const Store *>(B.pop[parity]), B.nbw, B.P, g,
-                                        p, b - first[l]);
+  const Store *A = static_cast<const Store *>(B.pop[parity]);
+  if (SOLID && p.has_solid)
+    ssplit_psi_block<Store, SOLID, OFF32>(A, B.nbw, B.P, g, p, b - first[l]);
+  else
+    ssplit_psi_block<Store, false, OFF32>(A, B.nbw, B.P, g, p, b - first[l]);
 }
 
 // ONE: both passes in one launch; q.order holds each turn and its lattice.
@@ -405,13 +411,15 @@ __global__ void __launch_bounds__(kShiftThreads) __attribute__((amdgpu_waves_per
       return;
     }
   }
-  ssplit_collide_block<Store, SOLID, OFF32>(
-      A, static_cast<Store *>(const_cast<void *>(B.pop[parity ^ 1])), B.nbw, B.P, g, p, b - f0,
-      nullptr);
+  Store *W = static_cast<Store *>(const_cast<void *>(B.pop[parity ^ 1]));
+  if (SOLID && (ONE || p.has_solid))
+    ssplit_collide_block<Store, SOLID, OFF32>(A, W, B.nbw, B.P, g, p, b - f0, nullptr);
+  else
+    ssplit_collide_block<Store, false, OFF32>(A, W, B.nbw, B.P, g, p, b - f0, nullptr);
 }
 
 // The split pair as one persistent launch per step: the workgroups (all
-// resident: a cooperative launch) take the 128-site blocks of every member in
+// resident: a cooperative launch) take the 256-site blocks of every member in
 // turn (block b on workgroup b mod G, so on the XCD the two-launch form runs
 // it on) for the psi pass, wait at a grid barrier, then take them again for
 // the stream/force/collide pass.  Same per-block code, hence the same bits,
