@@ -577,11 +577,11 @@ struct MarchStep {
 
 int effective_schedule(const dlbc_gpu_ctx *c) {
   if (c->schedule != DLBC_SCHED_AUTO) return c->schedule;
-  // shifted storage: the split kernels (256^3 channel: FP32 1.25 against 2.40 ms,
-  // FP16 0.84 against 2.0); the tiled kernel (FUSED) remains selectable
+  // shifted storage: the split kernels (256^3 channel: FP32 1.23 against 2.39 ms,
+  // FP16 0.84 against 2.07); the tiled kernel (FUSED) remains selectable
   if (c->storage != DLBC_STORAGE_F64) return DLBC_SCHED_SPLIT;
   // D3Q19 two-component FP64: the lane-per-component two-pass kernels are the
-  // fastest measured schedule (256^3 channel: 2.37 ms/step vs 4.20 ms fused)
+  // fastest measured schedule (256^3 channel: 2.42 ms/step vs 4.18 ms fused)
   if (c->d == 3 && c->C == 2) return DLBC_SCHED_SPLIT;
   return DLBC_SCHED_TWO_PASS;
 }
@@ -2059,7 +2059,7 @@ struct dlbc_batch {
                    // 3: the split pair as one persistent (cooperative) launch
   int coop_grid = 0;     // workgroups of that launch (0: not yet queried)
   int coop_variant = -1;  // the kernel variant coop_grid was queried for
-  int *d_first = nullptr;     // split: first 128-site block of each member, and the total
+  int *d_first = nullptr;     // split: first 256-site block of each member, and the total
   std::vector<int> h_first;
   // split pair in one launch: its turns (each with its lattice) and flags
   int32_t *order = nullptr;

@@ -125,7 +125,7 @@ int dlbc_gpu_step(dlbc_gpu_ctx *ctx, int nsteps);
 /* As dlbc_gpu_step, with the steps replayed from a captured HIP graph of 32
  * steps (one graph per buffer parity; the remainder of nsteps runs eagerly).
  * Same results bit for bit; for small lattices, whose steps are bound by
- * launch latency (two-fluid D3Q19 32^3: 9.8 instead of 10.6 us per step;
+ * launch latency (two-fluid D3Q19 32^3: 9.5 instead of 10.6 us per step;
  * single-component D2Q9, which takes up to eight steps per launch, is as fast
  * eagerly).  The graphs are
  * captured on first use and again when the schedule, launch shape, block
